@@ -41,34 +41,133 @@ namespace gapx {
 
 namespace {
 
+// FP64 elementary functions of the descriptor kernels, written for the
+// arguments these kernels have (no infinities, no range reduction beyond what
+// the formulas need), from minimax polynomials fitted with a Remez exchange.
+// (67,647 atoms, D = 128: the FP64 forward 1262 -> 1134 us.)
+// The library's exp costs about 30 vector instructions with its range checks,
+// its sincos about 70 (and much code for large arguments), its square root and
+// division about 17 and 11 with their scaling; these cost 18, 22, 11 and 5.
+//
+// The coefficients are kept in scalar registers (sconst): as plain literals
+// each would be moved into a vector register again for its fused multiply-add,
+// about ten more vector instructions per exponential.
+__device__ __forceinline__ double sconst(double c) {
+  asm("" : "+s"(c));
+  return c;
+}
+
+// exp(y): y = n ln2 + r, |r| <= ln2 / 2, 1 + r + r^2 q(r) with q of degree 9
+// (fit error 3.4e-18), scaled by 2^n.  Underflows to 0 and overflows to
+// infinity through the scaling; y must be finite.
+__device__ __forceinline__ double exp64(double y) {
+  const double n = __builtin_rint(y * sconst(1.4426950408889634));
+  double r = fma(n, sconst(-6.93147180559945286e-01), y);
+  r = fma(n, sconst(-2.31904681384629956e-17), r);
+  double q = sconst(2.5117915126746086e-08);
+  q = fma(q, r, sconst(2.76313397049011e-07));
+  q = fma(q, r, sconst(2.755721613139287e-06));
+  q = fma(q, r, sconst(2.480148978582598e-05));
+  q = fma(q, r, sconst(0.00019841269917571867));
+  q = fma(q, r, sconst(0.0013888888947156122));
+  q = fma(q, r, sconst(0.008333333333307118));
+  q = fma(q, r, sconst(0.04166666666651493));
+  q = fma(q, r, sconst(0.166666666666667));
+  q = fma(q, r, sconst(0.5000000000000013));
+  q = fma(q, r, 1.0);
+  q = fma(q, r, 1.0);
+  return __builtin_amdgcn_ldexp(q, (int)n);
+}
+
+// Cosine and sine of x = w r in [0, pi] (up to 1e-4 beyond), as -sin and cos
+// of y = x - pi/2: odd and even polynomials in y (fit errors 2e-19, 6e-18).
+__device__ __forceinline__ double quarter_shift(double w, double r) {
+  return fma(w, r, sconst(-1.57079632679489656)) + sconst(-6.12323399573676604e-17);
+}
+__device__ __forceinline__ double sin_quarter(double y, double z) {
+  double s = sconst(2.7184781158758493e-15);
+  s = fma(s, z, sconst(-7.642711170741734e-13));
+  s = fma(s, z, sconst(1.6058927767606374e-10));
+  s = fma(s, z, sconst(-2.5052106605227996e-08));
+  s = fma(s, z, sconst(2.7557319207770882e-06));
+  s = fma(s, z, sconst(-0.00019841269841185862));
+  s = fma(s, z, sconst(0.008333333333333113));
+  s = fma(s, z, sconst(-0.16666666666666666));
+  return fma(y * z, s, y);
+}
+__device__ __forceinline__ double cos_quarter(double z) {
+  double c = sconst(4.616102920731384e-14);
+  c = fma(c, z, sconst(-1.1463632624429262e-11));
+  c = fma(c, z, sconst(2.0876592494655193e-09));
+  c = fma(c, z, sconst(-2.7557317066796995e-07));
+  c = fma(c, z, sconst(2.4801587285768175e-05));
+  c = fma(c, z, sconst(-0.0013888888888829978));
+  c = fma(c, z, sconst(0.04166666666666583));
+  return fma(z * z, c, fma(-0.5, z, 1.0));
+}
+
+// 1 / x from the hardware estimate and two Newton steps.
+__device__ __forceinline__ double rcp64(double x) {
+  double v = __builtin_amdgcn_rcp(x);
+  v = fma(v, fma(-x, v, 1.0), v);
+  return fma(v, fma(-x, v, 1.0), v);
+}
+
 template <typename T>
 struct Math;
 
+// sqrt_rsq: e = sqrt(x) and i = 1 / e for x >= floor2().  cos1: 1 + cos(w r)
+// for w r in [0, pi]; sincos1 also the sine, with w from turn().
 template <>
 struct Math<double> {
-  static __device__ __forceinline__ double ex(double x) { return exp(x); }
-  static __device__ __forceinline__ double cs(double x) { return cos(x); }
-  static __device__ __forceinline__ double sn(double x) { return sin(x); }
-  // sine and cosine of one argument with one argument reduction
-  static __device__ __forceinline__ void sc(double x, double &s, double &c) { sincos(x, &s, &c); }
-  static __device__ __forceinline__ double sq(double x) { return sqrt(x); }
+  static __device__ __forceinline__ double ex(double x) { return exp64(x); }
+  static constexpr __device__ __forceinline__ double floor2() { return 1e-200; }
+  static __device__ __forceinline__ double turn(double pirc) { return pirc; }
+  static __device__ __forceinline__ void sqrt_rsq(double x, double &e, double &i) {
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    double d = fma(-h, g, 0.5);
+    g = fma(g, d, g);
+    h = fma(h, d, h);
+    e = fma(fma(-g, g, x), h, g);
+    h = fma(h, fma(-h, e, 0.5), h);
+    i = h + h;
+  }
+  static __device__ __forceinline__ double sq(double x) {
+    double e, i;
+    sqrt_rsq(fmax(x, floor2()), e, i);
+    return e;
+  }
+  static __device__ __forceinline__ double cos1(double w, double r) {
+    const double y = quarter_shift(w, r);
+    return 1.0 - sin_quarter(y, y * y);
+  }
+  static __device__ __forceinline__ void sincos1(double w, double r, double &s, double &c1) {
+    const double y = quarter_shift(w, r), z = y * y;
+    s = cos_quarter(z);
+    c1 = 1.0 - sin_quarter(y, z);
+  }
   static __device__ __forceinline__ double pw(double b, double e) { return pow(b, e); }
-  static __device__ __forceinline__ double rcp(double x) { return 1.0 / x; }
 };
 
 template <>
 struct Math<float> {
   static __device__ __forceinline__ float ex(float x) { return __expf(x); }
-  static __device__ __forceinline__ float cs(float x) { return __cosf(x); }
-  static __device__ __forceinline__ float sn(float x) { return __sinf(x); }
-  static __device__ __forceinline__ void sc(float x, float &s, float &c) {
-    s = __sinf(x);
-    c = __cosf(x);
+  static constexpr __device__ __forceinline__ float floor2() { return 1e-30f; }
+  // v_sin_f32 and v_cos_f32 take revolutions
+  static __device__ __forceinline__ float turn(float pirc) { return pirc * 0.159154943091895f; }
+  static __device__ __forceinline__ void sqrt_rsq(float x, float &e, float &i) {
+    i = __builtin_amdgcn_rsqf(x);
+    e = x * i;
   }
   static __device__ __forceinline__ float sq(float x) { return __builtin_amdgcn_sqrtf(x); }
+  static __device__ __forceinline__ float cos1(float w, float r) { return __cosf(w * r) + 1.f; }
+  static __device__ __forceinline__ void sincos1(float w, float r, float &s, float &c1) {
+    const float x = w * r;
+    s = __builtin_amdgcn_sinf(x);
+    c1 = __builtin_amdgcn_cosf(x) + 1.f;
+  }
   static __device__ __forceinline__ float pw(float b, float e) { return powf(b, e); }
-  // hardware approximations (about 1 ulp) for the mixed path's inner loops
-  static __device__ __forceinline__ float rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 };
 
 // Two values of T read as one LDS access (the backward's per-neighbour pairs).
@@ -83,6 +182,11 @@ struct Pair<double> {
   typedef double2 type;
 };
 
+template <typename T>
+struct alignas(16) Quad {
+  T v[4];
+};
+
 // A radial-table entry in the kernel's precision: the FP32 copy for FP32
 // kernels (the same rounding as converting the FP64 entry, without a
 // conversion per line and lane).
@@ -93,6 +197,10 @@ __device__ __forceinline__ T rad_table(const double *t64, const float *t32, int 
   else
     return t64[s];
 }
+
+// This wave's index in its workgroup, known uniform to the compiler: tables
+// indexed by it are then read with scalar loads.
+__device__ __forceinline__ int wave_index() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6); }
 
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
@@ -170,12 +278,45 @@ __device__ __forceinline__ double slot_weight(const NeighborBufs &nb, const doub
 }
 
 // Launch geometry of the descriptor kernels: LDS layout (neighbour slots,
-// cutoff groups, padded features) and the first atom of the launch (one
-// workgroup per atom from atom0 on).
+// cutoff groups, padded features, radial lines) and the first atom of the
+// launch (one workgroup per atom from atom0 on).
 struct Lds {
   int KP, G, Dp;
   int atom0;
+  int n_rad;
 };
+
+// Stage an atom's K neighbours in LDS: d = (dx, dy, dz, r), rw = (1 / r,
+// weight) and per cutoff group g, at row g KP, the cutoff function fc(r), or
+// with DERIV the pairs (fc, dfc/dr).  Threads tid, tid + nthr, ..
+template <typename T, bool DERIV>
+__device__ __forceinline__ void stage_neighbours(const NeighborBufs &nb, const double *wz, const int *species,
+                                                 const SFDev &sf, int start, int K, int KP, T *s_d, T *s_rw, T *s_fc,
+                                                 int tid, int nthr) {
+  for (int a = tid; a < K; a += nthr) {
+    const double2 *dd = (const double2 *)(nb.nb_d + 4 * (size_t)(start + a));
+    const double2 xy = dd[0], zr = dd[1];
+    const double r = zr.y;
+    s_d[4 * a] = (T)xy.x;
+    s_d[4 * a + 1] = (T)xy.y;
+    s_d[4 * a + 2] = (T)zr.x;
+    s_d[4 * a + 3] = (T)r;
+    s_rw[2 * a] = (T)rcp64(r);
+    s_rw[2 * a + 1] = (T)slot_weight(nb, wz, species, start + a);
+    for (int g = 0; g < sf.n_groups; ++g) {
+      const bool in = r <= sf.group_rc[g];
+      const double w = sf.group_pirc[g];
+      if constexpr (DERIV) {
+        double sn, c1;
+        Math<double>::sincos1(w, r, sn, c1);
+        s_fc[2 * (g * KP + a)] = in ? (T)(0.5 * c1) : T(0);
+        s_fc[2 * (g * KP + a) + 1] = in ? (T)(-0.5 * sn * w) : T(0);
+      } else {
+        s_fc[g * KP + a] = in ? (T)(0.5 * Math<double>::cos1(w, r)) : T(0);
+      }
+    }
+  }
+}
 
 // Triplet indices of wave steps t, t + stride, .. (4 steps) for one lane; the
 // loads are issued together, one iteration ahead of their use, so a wave
@@ -203,7 +344,7 @@ __device__ __forceinline__ uint32_t pop_q4(uint32_t (&q)[4]) {
 // ---------------------------------------------------------------------------
 template <typename T, int NCH>
 __device__ __forceinline__ void ang_fwd_term(uint32_t q, bool active, int c0, const SFDev &sf, const T *s_d,
-                                             const T *s_w, const T *s_fc, int KP, T (&acc)[NCH],
+                                             const T *s_rw, const T *s_fc, int KP, T (&acc)[NCH],
                                              T (&accw)[NCH]) {
   const int a = q & 0xffff, b = q >> 16;
   const T ax = s_d[4 * a], ay = s_d[4 * a + 1], az = s_d[4 * a + 2], ra = s_d[4 * a + 3];
@@ -211,9 +352,11 @@ __device__ __forceinline__ void ang_fwd_term(uint32_t q, bool active, int c0, co
   const T ex = bx - ax, ey = by - ay, ez = bz - az;
   const T e2 = ex * ex + ey * ey + ez * ez;
   const T e = Math<T>::sq(e2);
-  const T cth = (ra * ra + rb * rb - e2) / (T(2) * ra * rb);
+  typedef typename Pair<T>::type P2;
+  const P2 rwa = ((const P2 *)s_rw)[a], rwb = ((const P2 *)s_rw)[b];  // (1/r, w)
+  const T cth = (ra * ra + rb * rb - e2) * (T(0.5) * rwa.x * rwb.x);
   const T S2 = ra * ra + rb * rb + e2;
-  const T wab = s_w[a] * s_w[b];
+  const T wab = rwa.y * rwb.y;
   const T on = active ? T(1) : T(0);
   int cur_g = -1;
   T F3 = 0, E = 0, cur_eta = T(-1);
@@ -227,7 +370,7 @@ __device__ __forceinline__ void ang_fwd_term(uint32_t q, bool active, int c0, co
         cur_g = g;
         cur_eta = T(-1);  // E below carries this group's cutoff product
         const T rc = (T)sf.group_rc[g];
-        const T fe = (e <= rc) ? T(0.5) * (Math<T>::cs((T)kPi * e / rc) + T(1)) : T(0);
+        const T fe = (e <= rc) ? T(0.5) * Math<T>::cos1((T)sf.group_pirc[g], e) : T(0);
         F3 = s_fc[g * KP + a] * s_fc[g * KP + b] * fe * on;
       }
       const T eta = (T)sf.ang_eta[s];
@@ -276,20 +419,20 @@ __device__ __forceinline__ void chunk_reduce(T (&acc)[NCH], T (&accw)[NCH], int 
 // (row of atom i) instead of LDS, for neighbour lists too long for the LDS
 // layout (launched with one wavefront per atom).
 template <typename T, int NCH, int W, bool FG>
-__global__ __launch_bounds__(256) void k_desc_fwd(int N, const int *__restrict__ species,
+__global__ __launch_bounds__(W > 4 ? 64 * W : 256) void k_desc_fwd(int N, const int *__restrict__ species,
                                                   const double *__restrict__ wz, NeighborBufs nb, TripletBufs tb,
                                                   SFDev sf, Lds L, const double *__restrict__ theta_inv,
                                                   const double *__restrict__ mu, int split_mode, DescOut out) {
   extern __shared__ __align__(16) unsigned char smem[];
   if ((int)blockIdx.x >= N) return;  // one workgroup per atom of [atom0, atom0 + N)
   const int i = L.atom0 + blockIdx.x;
-  const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wv = wave_index(), lane = tid & 63;
   const int KP = L.KP, Dp = L.Dp;
-  double *s_xn = (double *)smem;  // [W]
-  T *s_d = (T *)(s_xn + W);
-  T *s_w = s_d + 4 * KP;
-  T *s_fc = FG ? (T *)nb.fc_scratch + (size_t)i * L.G * KP : s_w + KP;
-  T *s_feat = FG ? s_w + KP : s_fc + L.G * KP;
+  double *s_xn = (double *)smem;  // [W], padded to 16 bytes
+  T *s_d = (T *)(s_xn + ((W + 1) & ~1));
+  T *s_rw = s_d + 4 * KP;         // [KP] pairs (1 / r, species weight)
+  T *s_fc = FG ? (T *)nb.fc_scratch + (size_t)i * L.G * KP : s_rw + 2 * KP;
+  T *s_feat = FG ? s_rw + 2 * KP : s_fc + L.G * KP;
   T *s_part = s_feat + Dp;  // [W * 2 * NCH]
 
   const int start = i * nb.kcap;
@@ -298,19 +441,7 @@ __global__ __launch_bounds__(256) void k_desc_fwd(int N, const int *__restrict__
     if (tid == 0) atomicAdd(&nb.total[3], 1);
     return;
   }
-  for (int a = tid; a < K; a += 64 * W) {
-    const double *dd = nb.nb_d + 4 * (size_t)(start + a);
-    const double r = dd[3];
-    s_d[4 * a] = (T)dd[0];
-    s_d[4 * a + 1] = (T)dd[1];
-    s_d[4 * a + 2] = (T)dd[2];
-    s_d[4 * a + 3] = (T)r;
-    s_w[a] = (T)slot_weight(nb, wz, species, start + a);
-    for (int g = 0; g < sf.n_groups; ++g) {
-      const double rc = sf.group_rc[g];
-      s_fc[g * KP + a] = (r <= rc) ? (T)(0.5 * (cos(kPi * r / rc) + 1.0)) : T(0);
-    }
-  }
+  stage_neighbours<T, false>(nb, wz, species, sf, start, K, KP, s_d, s_rw, s_fc, tid, 64 * W);
   for (int d = tid; d < Dp; d += 64 * W) s_feat[d] = T(0);
   __syncthreads();
 
@@ -320,7 +451,7 @@ __global__ __launch_bounds__(256) void k_desc_fwd(int N, const int *__restrict__
 #pragma unroll
     for (int l = 0; l < NCH; ++l) acc[l] = accw[l] = T(0);
     for (int a = tid; a < K; a += 64 * W) {
-      const T r = s_d[4 * a + 3], w = s_w[a];
+      const T r = s_d[4 * a + 3], w = s_rw[2 * a + 1];
 #pragma unroll
       for (int l = 0; l < NCH; ++l) {
         const int s = c0 + l;
@@ -350,7 +481,7 @@ __global__ __launch_bounds__(256) void k_desc_fwd(int N, const int *__restrict__
 #pragma unroll 1
       for (int u = 0; u < 4; ++u) {
         const uint32_t q = pop_q4(qc);
-        ang_fwd_term<T, NCH>(q, t0 + u * ST + lane < nt, c0, sf, s_d, s_w, s_fc, KP, acc, accw);
+        ang_fwd_term<T, NCH>(q, t0 + u * ST + lane < nt, c0, sf, s_d, s_rw, s_fc, KP, acc, accw);
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) qc[u] = qn[u];
@@ -409,7 +540,9 @@ __global__ __launch_bounds__(256) void k_desc_fwd(int N, const int *__restrict__
 // Z16: the zeta list is {1, 2, 4, 16} (zlog {0, 1, 2, 4}, the usual grid),
 // known at compile time, so the chain is straight-line code with the same
 // multiplications in the same order.
-template <typename T, int NZ, bool DERIV, bool Z16>
+// RAWQ: dPp and dPm are the bare u^(zeta_k - 1) (the callers carry the factors
+// lam zeta_k / 2 elsewhere).
+template <typename T, int NZ, bool DERIV, bool Z16, bool RAWQ = false>
 __device__ __forceinline__ void grid_powers(T cth, const SFDev &sf, T (&Pp)[NZ], T (&Pm)[NZ], T (&dPp)[NZ],
                                             T (&dPm)[NZ]) {
   static_assert(!Z16 || NZ == 4, "the {1, 2, 4, 16} list has four zetas");
@@ -445,24 +578,29 @@ __device__ __forceinline__ void grid_powers(T cth, const SFDev &sf, T (&Pp)[NZ],
     Pp[k] = p;
     Pm[k] = m;
     if (DERIV) {
-      const T hz = T(0.5) * (T)sf.zeta_k[k];  // zeta_k / 2, exact
-      dPp[k] = hz * qp;
-      dPm[k] = -hz * qm;
+      const T hz = RAWQ ? T(1) : T(0.5) * (T)sf.zeta_k[k];  // zeta_k / 2, exact
+      dPp[k] = RAWQ ? qp : hz * qp;
+      dPm[k] = RAWQ ? qm : -hz * qm;
     }
   }
 }
 
 // exp(-eta x) as the grid kernels evaluate it: in FP32 the hardware 2^x with
 // the coefficient -eta log2(e) formed once per eta (one multiplication per
-// term instead of two); in FP64 exp itself.
+// term instead of two); in FP64 exp64.
 template <typename T>
 __device__ __forceinline__ T eta_coef(T eta);
 template <>
 __device__ __forceinline__ float eta_coef<float>(float eta) { return -eta * 1.44269504088896341f; }
 template <>
 __device__ __forceinline__ double eta_coef<double>(double eta) { return -eta; }
+// 2 A / |coefficient|: the factor that turns coefficient times dr into -2 A dr.
+template <typename T>
+constexpr __device__ __forceinline__ T slope_factor() {
+  return sizeof(T) == 4 ? T(1.38629436111989062) : T(2);
+}
 __device__ __forceinline__ float exp_coef(float c, float x) { return __builtin_amdgcn_exp2f(c * x); }
-__device__ __forceinline__ double exp_coef(double c, double x) { return exp(c * x); }
+__device__ __forceinline__ double exp_coef(double c, double x) { return exp64(c * x); }
 
 // Sum NV per-lane values over the workgroup: s_out[j] = total of v[j].  Within
 // a wavefront a butterfly reduce-scatter: at offset m (32, 16, .., 1) every
@@ -530,23 +668,31 @@ __device__ __forceinline__ void butterfly(T (&x)[NVP], int lane) {
   }
 }
 
-template <typename T, int NV, int W>
-__device__ __forceinline__ void group_sum(T (&v)[NV], int wv, int lane, int tid, T *s_part, T *s_out) {
-  constexpr int NVP = NV <= 32 ? 32 : 64;
+// Within the wave: lane l returns the total of v[l % NVP], NVP the next power
+// of two (8 to 64) from NV; with fewer than 64 values the butterfly (offsets
+// NVP / 2 .. 1) stays within NVP lanes and the groups' totals are added last.
+template <typename T, int NV>
+__device__ __forceinline__ T wave_totals(T (&v)[NV], int lane) {
   static_assert(NV <= 64, "at most 64 values");
+  constexpr int NVP = NV <= 8 ? 8 : NV <= 16 ? 16 : NV <= 32 ? 32 : 64;
   T x[NVP];
 #pragma unroll
   for (int j = 0; j < NVP; ++j) x[j] = (j < NV) ? v[j] : T(0);
   butterfly<T, NVP / 2, NVP>(x, lane);
-  // 32 values: the butterfly (offsets 16 .. 1) stays within each half of
-  // the wave; lanes l and l + 32 then add their halves' totals of value l
-  if (NVP == 32) x[0] += __shfl_xor(x[0], 32, 64);
+#pragma unroll
+  for (int o = NVP; o < 64; o <<= 1) x[0] += __shfl_xor(x[0], o, 64);
+  return x[0];
+}
+
+template <typename T, int NV, int W>
+__device__ __forceinline__ void group_sum(T (&v)[NV], int wv, int lane, int tid, T *s_part, T *s_out) {
+  const T x = wave_totals<T, NV>(v, lane);
   if (W == 1) {
-    if (lane < NV) s_out[lane] = x[0];
+    if (lane < NV) s_out[lane] = x;
     __syncthreads();
     return;
   }
-  if (lane < NV) s_part[wv * NV + lane] = x[0];
+  if (lane < NV) s_part[wv * NV + lane] = x;
   __syncthreads();
   for (int j = tid; j < NV; j += 64 * W) {
     T sum = T(0);
@@ -565,17 +711,17 @@ struct GridShape {
 };
 
 template <typename T, int NZ, int W, bool Z16, bool FG>
-__global__ __launch_bounds__(256) void k_desc_fwd_grid(int N, const int *__restrict__ species,
+__global__ __launch_bounds__(W > 4 ? 64 * W : 256) void k_desc_fwd_grid(int N, const int *__restrict__ species,
                                                        const double *__restrict__ wz, NeighborBufs nb,
                                                        TripletBufs tb, SFDev sf, Lds L,
                                                        const double *__restrict__ theta_inv,
                                                        const double *__restrict__ mu, int split_mode, DescOut out) {
   constexpr int NE = GridShape<T, NZ>::NE, NV = GridShape<T, NZ>::NV;
-  constexpr int RCH = 16;
+  constexpr int RCH = W <= 2 ? 16 : 32 / W;  // radial lines per chunk
   extern __shared__ __align__(16) unsigned char smem[];
   if ((int)blockIdx.x >= N) return;  // one workgroup per atom of [atom0, atom0 + N)
   const int i = L.atom0 + blockIdx.x;
-  const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wv = wave_index(), lane = tid & 63;
   const int KP = L.KP, Dp = L.Dp;
   double *s_xn = (double *)smem;  // [W], padded to 16 bytes
   T *s_d = (T *)(s_xn + ((W + 1) & ~1));
@@ -591,31 +737,19 @@ __global__ __launch_bounds__(256) void k_desc_fwd_grid(int N, const int *__restr
     if (tid == 0) atomicAdd(&nb.total[3], 1);
     return;
   }
-  for (int a = tid; a < K; a += 64 * W) {
-    const double *dd = nb.nb_d + 4 * (size_t)(start + a);
-    const double r = dd[3];
-    s_d[4 * a] = (T)dd[0];
-    s_d[4 * a + 1] = (T)dd[1];
-    s_d[4 * a + 2] = (T)dd[2];
-    s_d[4 * a + 3] = (T)r;
-    s_rw[2 * a] = (T)(1.0 / r);
-    s_rw[2 * a + 1] = (T)slot_weight(nb, wz, species, start + a);
-    for (int g = 0; g < sf.n_groups; ++g) {
-      const double rc = sf.group_rc[g];
-      s_fc[g * KP + a] = (r <= rc) ? (T)(0.5 * (cos(kPi * r / rc) + 1.0)) : T(0);
-    }
-  }
+  stage_neighbours<T, false>(nb, wz, species, sf, start, K, KP, s_d, s_rw, s_fc, tid, 64 * W);
   for (int d = tid; d < Dp; d += 64 * W) s_feat[d] = T(0);
   __syncthreads();
 
-  // radial lines, RCH at a time: plain sums in acc[0, RCH), weighted ones in
-  // acc[RCH, 2 RCH), reduced over the group with the angular pass's exchange
-  static_assert(2 * RCH <= NV, "radial sums reuse the angular reduction buffers");
-  for (int c0 = 0; c0 < sf.n_rad; c0 += RCH) {
+  // radial lines, RCH at a time, each chunk by one wave over all neighbours:
+  // plain sums in acc[0, RCH), weighted ones in acc[RCH, 2 RCH), reduced
+  // within the wave (with W waves the chunks of a usual table run beside each
+  // other, and none needs an exchange between waves)
+  for (int c0 = wv * RCH; c0 < sf.n_rad; c0 += W * RCH) {
     T acc[2 * RCH];
 #pragma unroll
     for (int l = 0; l < 2 * RCH; ++l) acc[l] = T(0);
-    for (int a = tid; a < K; a += 64 * W) {
+    for (int a = lane; a < K; a += 64) {
       const T r = s_d[4 * a + 3], w = s_rw[2 * a + 1];
 #pragma unroll
       for (int l = 0; l < RCH; ++l) {
@@ -628,12 +762,9 @@ __global__ __launch_bounds__(256) void k_desc_fwd_grid(int N, const int *__restr
         }
       }
     }
-    group_sum<T, 2 * RCH, W>(acc, wv, lane, tid, s_part, s_sum);
-    for (int j = tid; j < 2 * RCH; j += 64 * W) {
-      const int l = j % RCH;
-      if (c0 + l < sf.n_rad) s_feat[sf.rad_feat[c0 + l] + (j >= RCH ? sf.nsf : 0)] = s_sum[j];
-    }
-    __syncthreads();
+    const T v = wave_totals<T, 2 * RCH>(acc, lane);
+    const int l = lane % RCH;
+    if (lane < 2 * RCH && c0 + l < sf.n_rad) s_feat[sf.rad_feat[c0 + l] + (lane >= RCH ? sf.nsf : 0)] = v;
   }
 
   // angular lines in grid form, NE etas per pass
@@ -641,7 +772,7 @@ __global__ __launch_bounds__(256) void k_desc_fwd_grid(int N, const int *__restr
   const int nt = tb.count[i];
   const int g = sf.g_ang;
   const T rc = (T)sf.group_rc[g];
-  const T pirc = (T)(kPi / sf.group_rc[g]);
+  const T pirc = (T)sf.group_pirc[g];
   for (int h0 = 0; h0 < sf.n_eta; h0 += NE) {
     T acc[NV];
 #pragma unroll
@@ -671,7 +802,7 @@ __global__ __launch_bounds__(256) void k_desc_fwd_grid(int N, const int *__restr
         const T S2 = ra * ra + rb * rb + e2;
         const T wab = rwa.y * rwb.y;
         // 2 fc(r_jk): the factor 2 of the halved powers (grid_powers) rides here
-        const T fe2 = (e <= rc) ? Math<T>::cs(pirc * e) + T(1) : T(0);
+        const T fe2 = (e <= rc) ? Math<T>::cos1(pirc, e) : T(0);
         const T F3 = act ? s_fc[g * KP + a] * s_fc[g * KP + b] * fe2 : T(0);
         T Pp[NZ], Pm[NZ], dPp[NZ], dPm[NZ];
         grid_powers<T, NZ, false, Z16>(cth, sf, Pp, Pm, dPp, dPm);
@@ -745,11 +876,114 @@ struct EtaRec {
   static constexpr int RS = NZ > 0 ? (4 * NZ + 2 + 3) & ~3 : 0;
 };
 
-template <typename T, int NZ, bool Z16>
+// The grid-form backward's per-eta sums over the 2 NZ lines,
+//   sb_h = sum_z (gA_hz + w gW_hz) P_z,   sa_h the same with dP_z / dcos,
+// need all 4 NZ values of g per eta for every triplet.  Read from LDS as
+// records (one address for the whole wave), those reads were 20 (FP32) to 36
+// (FP64) of the 34 to 50 LDS instructions per 64 triplets, and with the LDS
+// busy 72-79 % of the time they bounded the kernel; so g stays in registers
+// spread over the lanes, in the forms below.
+
+// FP32 on the matrix cores: v_mfma_f32_4x4x1_16b_f32 multiplies, in each of
+// 16 groups of four lanes, a column of four A values by a row of four B values.
+// With B = P_z of each lane's own triplet and A = g of four etas for line z
+// (held by the lanes 4 z .. 4 z + 3 of one register and broadcast to every group:
+// cbsz 4, abid z), lane l's four results are its own triplet's four partial
+// sums: no data moves between lanes, each is an FP32 fused multiply-add as
+// on the vector units, and 96 of the 220 vector instructions per 64 triplets
+// move to the otherwise idle matrix cores.
+typedef float v4f __attribute__((ext_vector_type(4)));
+
+// Registers of one set of four etas: lane 4 z + i holds line z of eta i, plain
+// (a) and weighted (w), for P (p) and, with the factor lam zeta / 2, for the
+// bare derivative powers (q).
+struct EtaSet {
+  float ap, wp, aq, wq;
+};
+
+template <int NZ>
+__device__ __forceinline__ EtaSet load_eta_set(const SFDev &sf, const float *s_g, int set, int lane) {
+  const int h = 4 * set + (lane & 3), z = lane >> 2;
+  EtaSet e{0.f, 0.f, 0.f, 0.f};
+  if (h < sf.n_eta && z < 2 * NZ) {
+    const int s = h * 2 * NZ + z, f = sf.ang_feat[s];
+    const float hz = (z < NZ ? 0.5f : -0.5f) * (float)sf.ang_zeta[s];
+    e.ap = s_g[f];
+    e.wp = s_g[f + sf.nsf];
+    e.aq = hz * e.ap;
+    e.wq = hz * e.wp;
+  }
+  return e;
+}
+
+template <int Z, int NZ>
+__device__ __forceinline__ void eta_products(const EtaSet &e, const float (&Pp)[NZ], const float (&Pm)[NZ],
+                                             const float (&Qp)[NZ], const float (&Qm)[NZ], v4f &ba, v4f &bw, v4f &aa,
+                                             v4f &aw) {
+  if constexpr (Z < 2 * NZ) {
+    constexpr int k = Z % NZ;
+    const float P = Z < NZ ? Pp[k] : Pm[k], Q = Z < NZ ? Qp[k] : Qm[k];
+    ba = __builtin_amdgcn_mfma_f32_4x4x1f32(e.ap, P, ba, 4, Z, 0);
+    bw = __builtin_amdgcn_mfma_f32_4x4x1f32(e.wp, P, bw, 4, Z, 0);
+    aa = __builtin_amdgcn_mfma_f32_4x4x1f32(e.aq, Q, aa, 4, Z, 0);
+    aw = __builtin_amdgcn_mfma_f32_4x4x1f32(e.wq, Q, aw, 4, Z, 0);
+    eta_products<Z + 1, NZ>(e, Pp, Pm, Qp, Qm, ba, bw, aa, aw);
+  }
+}
+
+// FP64 through the cross-lane operand of the vector units: a row of 16 lanes
+// holds an eta's line values, line z in lane z, and v_fmac_f64 takes one of
+// them, broadcast over the row (row_newbcast), as its multiplicand.  A block
+// does lines Z .. Z + NB - 1; its first instruction waits out the two states
+// between a vector write of a register and its cross-lane read.
+#define GAPX_ROW_LINE(z, p, q)                                    \
+  "v_fmac_f64_dpp %0, %4, " p " row_newbcast:" z " row_mask:0xf bank_mask:0xf\n" \
+  "v_fmac_f64_dpp %1, %5, " p " row_newbcast:" z " row_mask:0xf bank_mask:0xf\n" \
+  "v_fmac_f64_dpp %2, %4, " q " row_newbcast:" z " row_mask:0xf bank_mask:0xf\n" \
+  "v_fmac_f64_dpp %3, %5, " q " row_newbcast:" z " row_mask:0xf bank_mask:0xf\n"
+template <int Z, int NZ>
+__device__ __forceinline__ void row_products(double ga, double gw, const double (&Pp)[NZ], const double (&Pm)[NZ],
+                                             const double (&dPp)[NZ], const double (&dPm)[NZ], double &ba, double &bw,
+                                             double &aa, double &aw) {
+  static_assert(2 * NZ <= 16, "a row has 16 lanes");
+  auto P = [&](int z) { return z < NZ ? Pp[z] : Pm[z - NZ]; };
+  auto Q = [&](int z) { return z < NZ ? dPp[z] : dPm[z - NZ]; };
+  if constexpr (Z + 4 <= 2 * NZ) {
+    asm("s_nop 1\n" GAPX_ROW_LINE("%c14", "%6", "%10") GAPX_ROW_LINE("%c15", "%7", "%11")
+            GAPX_ROW_LINE("%c16", "%8", "%12") GAPX_ROW_LINE("%c17", "%9", "%13")
+        : "+&v"(ba), "+&v"(bw), "+&v"(aa), "+&v"(aw)
+        : "v"(ga), "v"(gw), "v"(P(Z)), "v"(P(Z + 1)), "v"(P(Z + 2)), "v"(P(Z + 3)), "v"(Q(Z)), "v"(Q(Z + 1)),
+          "v"(Q(Z + 2)), "v"(Q(Z + 3)), "i"(Z), "i"(Z + 1), "i"(Z + 2), "i"(Z + 3));
+    row_products<Z + 4, NZ>(ga, gw, Pp, Pm, dPp, dPm, ba, bw, aa, aw);
+  } else if constexpr (Z + 2 <= 2 * NZ) {
+    asm("s_nop 1\n" GAPX_ROW_LINE("%c10", "%6", "%8") GAPX_ROW_LINE("%c11", "%7", "%9")
+        : "+&v"(ba), "+&v"(bw), "+&v"(aa), "+&v"(aw)
+        : "v"(ga), "v"(gw), "v"(P(Z)), "v"(P(Z + 1)), "v"(Q(Z)), "v"(Q(Z + 1)), "i"(Z), "i"(Z + 1));
+    row_products<Z + 2, NZ>(ga, gw, Pp, Pm, dPp, dPm, ba, bw, aa, aw);
+  }
+}
+#undef GAPX_ROW_LINE
+
+// g of the grid-form backward in registers, for tables of at most 4 ES etas
+// (ES > 0: FP32 up to two sets, FP64 one); ES = 0: from the LDS records.
+template <typename T, int ES>
+struct EtaRegs;
+template <int ES>
+struct EtaRegs<float, ES> {
+  EtaSet set[ES > 0 ? ES : 1];
+};
+template <int ES>
+struct EtaRegs<double, ES> {
+  double ga[4], gw[4];  // row lane z: line z of eta h
+};
+
+template <typename T, int NZ, bool Z16, int ES>
 __device__ __forceinline__ void ang_bwd_grid(uint32_t q, bool active, const SFDev &sf, const T *s_d, const T *s_rw,
-                                             const T *s_fd, const T *s_er, int KP, T rc, T pirc, double *s_T,
-                                             double *s_F) {
-  if (!active) return;
+                                             const T *s_fd, const T *s_er, const EtaRegs<T, ES> &er,
+                                             const T (&ceta)[4 * ES + 1], const T (&eta)[4 * ES + 1], int KP, T rc,
+                                             T pirc, double *s_T, double *s_F) {
+  // idle lanes work on neighbours 0 and 1 (the products need every lane) and
+  // add nothing at the end
   const int a = q & 0xffff, b = q >> 16;
   const T ax = s_d[4 * a], ay = s_d[4 * a + 1], az = s_d[4 * a + 2], ra = s_d[4 * a + 3];
   const T bx = s_d[4 * b], by = s_d[4 * b + 1], bz = s_d[4 * b + 2], rb = s_d[4 * b + 3];
@@ -757,8 +991,10 @@ __device__ __forceinline__ void ang_bwd_grid(uint32_t q, bool active, const SFDe
   const P2 rwa = ((const P2 *)s_rw)[a], rwb = ((const P2 *)s_rw)[b];  // (1/r, w)
   const T ria = rwa.x, rib = rwb.x;
   const T ex = bx - ax, ey = by - ay, ez = bz - az;
-  const T e2 = ex * ex + ey * ey + ez * ez;
-  const T e = Math<T>::sq(e2);
+  // the floor keeps 1 / e finite for coincident neighbours (their vector is 0)
+  const T e2 = fma(ex, ex, fma(ey, ey, fma(ez, ez, Math<T>::floor2())));
+  T e, ie;
+  Math<T>::sqrt_rsq(e2, e, ie);
   const T inv2ab = T(0.5) * ria * rib;
   const T cth = (ra * ra + rb * rb - e2) * inv2ab;
   const T S2 = ra * ra + rb * rb + e2;
@@ -768,68 +1004,69 @@ __device__ __forceinline__ void ang_bwd_grid(uint32_t q, bool active, const SFDe
   const P2 fda = ((const P2 *)s_fd)[g * KP + a], fdb = ((const P2 *)s_fd)[g * KP + b];  // (fc, dfc)
   const T fa = fda.x, dfa = fda.y, fb = fdb.x, dfb = fdb.y;
   const bool in = e <= rc;
-  T sine, cosine;
-  Math<T>::sc(pirc * e, sine, cosine);
+  T sine, cos1;
+  Math<T>::sincos1(Math<T>::turn(pirc), e, sine, cos1);
   // 2 fc(r_jk) and its derivative: every term below carries exactly one of
   // them, which puts the factor 2 of the halved powers (grid_powers) on all
-  const T fe = in ? cosine + T(1) : T(0);
+  const T fe = in ? cos1 : T(0);
   const T dfe = in ? -sine * pirc : T(0);
   T Pp[NZ], Pm[NZ], dPp[NZ], dPm[NZ];
-  grid_powers<T, NZ, true, Z16>(cth, sf, Pp, Pm, dPp, dPm);
+  constexpr bool kMfma = ES > 0 && sizeof(T) == 4;
+  grid_powers<T, NZ, true, Z16, kMfma>(cth, sf, Pp, Pm, dPp, dPm);
   T SA = 0, SB = 0, SC = 0;
-  // one eta: the lines' g contracted with the powers (sb) and with their
-  // cos-derivatives (sa), each sum started from its first term
-  auto eta_terms = [&](int h) {
-    const T *rec = s_er + h * EtaRec<NZ>::RS;
-    const T eta = rec[4 * NZ];
-    const T E = exp_coef(rec[4 * NZ + 1], S2);
-    T gA[2 * NZ], gW[2 * NZ];
-    if constexpr (sizeof(T) == 4 && NZ % 2 == 0) {
-      // 16-byte reads: records and both blocks are aligned
-      const float4 *a4 = (const float4 *)rec, *w4 = (const float4 *)(rec + 2 * NZ);
-#pragma unroll
-      for (int v = 0; v < NZ / 2; ++v) {
-        const float4 x = a4[v], y = w4[v];
-        gA[4 * v] = x.x, gA[4 * v + 1] = x.y, gA[4 * v + 2] = x.z, gA[4 * v + 3] = x.w;
-        gW[4 * v] = y.x, gW[4 * v + 1] = y.y, gW[4 * v + 2] = y.z, gW[4 * v + 3] = y.w;
-      }
-    } else {
-#pragma unroll
-      for (int j = 0; j < 2 * NZ; ++j) {
-        gA[j] = rec[j];
-        gW[j] = rec[2 * NZ + j];
-      }
-    }
-    // one fused multiply-add per term (a sum of term pairs would cost a
-    // multiply, an fma and an add per pair)
-    const T gp0 = gA[0] + wab * gW[0], gm0 = gA[NZ] + wab * gW[NZ];
-    T sa = gp0 * dPp[0];
-    T sb = gp0 * Pp[0];
-    sa = fma(gm0, dPm[0], sa);
-    sb = fma(gm0, Pm[0], sb);
-#pragma unroll
-    for (int k = 1; k < NZ; ++k) {
-      const T gp = gA[k] + wab * gW[k];
-      const T gm = gA[NZ + k] + wab * gW[NZ + k];
-      sa = fma(gp, dPp[k], sa);
-      sb = fma(gp, Pp[k], sb);
-      sa = fma(gm, dPm[k], sa);
-      sb = fma(gm, Pm[k], sb);
-    }
+  // one eta's sums over the lines times its exponential
+  auto add_eta = [&](T sa, T sb, T E, T et) {
+    const T t = sb * E;
     SA += sa * E;
-    SB += sb * E;
-    SC += eta * sb * E;
+    SB += t;
+    SC += et * t;
   };
-  for (int h = 0; h < sf.n_eta; ++h) eta_terms(h);
-  const T F = fa * fb * fe;
-  const T Ta = F * SA * dca - T(2) * ra * F * SC + SB * dfa * fb * fe;
-  const T Tb = F * SA * dcb - T(2) * rb * F * SC + SB * fa * dfb * fe;
-  const T Te = F * SA * dce - T(2) * e * F * SC + SB * fa * fb * dfe;
-  atomicAdd(&s_T[a], (double)Ta);
-  atomicAdd(&s_T[b], (double)Tb);
-  if (e > T(0)) {
-    const T sc = Te * Math<T>::rcp(e);
-    const T ux = sc * ex, uy = sc * ey, uz = sc * ez;
+  if constexpr (kMfma) {
+#pragma unroll
+    for (int u = 0; u < ES; ++u) {
+      v4f ba{0.f, 0.f, 0.f, 0.f}, bw = ba, aa = ba, aw = ba;
+      eta_products<0, NZ>(er.set[u], Pp, Pm, dPp, dPm, ba, bw, aa, aw);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        add_eta(aa[i] + wab * aw[i], ba[i] + wab * bw[i], exp_coef(ceta[4 * u + i], S2), eta[4 * u + i]);
+    }
+  } else if constexpr (ES > 0) {
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      if (h < sf.n_eta) {
+        T ba = 0, bw = 0, aa = 0, aw = 0;
+        row_products<0, NZ>(er.ga[h], er.gw[h], Pp, Pm, dPp, dPm, ba, bw, aa, aw);
+        add_eta(aa + wab * aw, ba + wab * bw, exp_coef(ceta[h], S2), eta[h]);
+      }
+    }
+  } else {
+    // from the LDS records: the lines' g contracted with the powers (sb) and
+    // with their cos-derivatives (sa), each sum started from its first term
+    for (int h = 0; h < sf.n_eta; ++h) {
+      const T *rec = s_er + h * EtaRec<NZ>::RS;
+      const T E = exp_coef(rec[4 * NZ + 1], S2);
+      T sa = 0, sb = 0;
+#pragma unroll
+      for (int k = 0; k < NZ; ++k) {
+        const T gp = rec[k] + wab * rec[2 * NZ + k];
+        const T gm = rec[NZ + k] + wab * rec[3 * NZ + k];
+        sa = k == 0 ? gp * dPp[0] : fma(gp, dPp[k], sa);
+        sb = k == 0 ? gp * Pp[0] : fma(gp, Pp[k], sb);
+        sa = fma(gm, dPm[k], sa);
+        sb = fma(gm, Pm[k], sb);
+      }
+      add_eta(sa, sb, E, rec[4 * NZ]);
+    }
+  }
+  const T F = fa * fb * fe, FA = F * SA, FC = T(-2) * F * SC;
+  const T Ta = FA * dca + ra * FC + SB * (dfa * (fb * fe));
+  const T Tb = FA * dcb + rb * FC + SB * (dfb * (fa * fe));
+  const T Te = FA * dce + e * FC + SB * (fa * fb * dfe);
+  const T sc = Te * ie;  // at e = 0 the vector is 0
+  const T ux = sc * ex, uy = sc * ey, uz = sc * ez;
+  if (active) {
+    atomicAdd(&s_T[a], (double)Ta);
+    atomicAdd(&s_T[b], (double)Tb);
     atomicAdd(&s_F[3 * b], (double)ux);
     atomicAdd(&s_F[3 * b + 1], (double)uy);
     atomicAdd(&s_F[3 * b + 2], (double)uz);
@@ -851,13 +1088,17 @@ __device__ __forceinline__ void ang_bwd_term(uint32_t q, bool active, const SFDe
   const T ax = s_d[4 * a], ay = s_d[4 * a + 1], az = s_d[4 * a + 2], ra = s_d[4 * a + 3];
   const T bx = s_d[4 * b], by = s_d[4 * b + 1], bz = s_d[4 * b + 2], rb = s_d[4 * b + 3];
   const T ex = bx - ax, ey = by - ay, ez = bz - az;
-  const T e2 = ex * ex + ey * ey + ez * ez;
-  const T e = Math<T>::sq(e2);
-  const T inv2ab = T(1) / (T(2) * ra * rb);
+  const T e2 = fma(ex, ex, fma(ey, ey, fma(ez, ez, Math<T>::floor2())));
+  T e, ie;
+  Math<T>::sqrt_rsq(e2, e, ie);
+  typedef typename Pair<T>::type P2;
+  const P2 rwa = ((const P2 *)s_rw)[a], rwb = ((const P2 *)s_rw)[b];  // (1/r, w)
+  const T ria = rwa.x, rib = rwb.x;
+  const T inv2ab = T(0.5) * ria * rib;
   const T cth = (ra * ra + rb * rb - e2) * inv2ab;
   const T S2 = ra * ra + rb * rb + e2;
-  const T dca = T(1) / rb - cth / ra, dcb = T(1) / ra - cth / rb, dce = -e * (T(2) * inv2ab);
-  const T wab = s_rw[2 * a + 1] * s_rw[2 * b + 1];
+  const T dca = rib - cth * ria, dcb = ria - cth * rib, dce = -e * (T(2) * inv2ab);
+  const T wab = rwa.y * rwb.y;
   T Ta = 0, Tb = 0, Te = 0;
   T SA = 0, SB = 0, SC = 0;
   T fa = 0, dfa = 0, fb = 0, dfb = 0, fe = 0, dfe = 0;
@@ -882,10 +1123,11 @@ __device__ __forceinline__ void ang_bwd_term(uint32_t q, bool active, const SFDe
       fb = s_fd[2 * (g * KP + b)];
       dfb = s_fd[2 * (g * KP + b) + 1];
       const bool in = e <= rc;
-      T sine, cosine;
-      Math<T>::sc((T)kPi * e / rc, sine, cosine);
-      fe = in ? T(0.5) * (cosine + T(1)) : T(0);
-      dfe = in ? T(0.5) * (-sine) * ((T)kPi / rc) : T(0);
+      const T pirc = (T)sf.group_pirc[g];
+      T sine, cos1;
+      Math<T>::sincos1(Math<T>::turn(pirc), e, sine, cos1);
+      fe = in ? T(0.5) * cos1 : T(0);
+      dfe = in ? T(-0.5) * sine * pirc : T(0);
     }
     const T eta = (T)sf.ang_eta[s];
     if (eta != cur_eta) {
@@ -903,49 +1145,78 @@ __device__ __forceinline__ void ang_bwd_term(uint32_t q, bool active, const SFDe
   if (cur_g >= 0) flush();
   atomicAdd(&s_T[a], (double)Ta);
   atomicAdd(&s_T[b], (double)Tb);
-  if (e > T(0)) {
-    const T s = Te / e;
-    const T ux = s * ex, uy = s * ey, uz = s * ez;
-    atomicAdd(&s_F[3 * b], (double)ux);
-    atomicAdd(&s_F[3 * b + 1], (double)uy);
-    atomicAdd(&s_F[3 * b + 2], (double)uz);
-    atomicAdd(&s_F[3 * a], (double)-ux);
-    atomicAdd(&s_F[3 * a + 1], (double)-uy);
-    atomicAdd(&s_F[3 * a + 2], (double)-uz);
-  }
+  const T s = Te * ie;
+  const T ux = s * ex, uy = s * ey, uz = s * ez;
+  atomicAdd(&s_F[3 * b], (double)ux);
+  atomicAdd(&s_F[3 * b + 1], (double)uy);
+  atomicAdd(&s_F[3 * b + 2], (double)uz);
+  atomicAdd(&s_F[3 * a], (double)-ux);
+  atomicAdd(&s_F[3 * a + 1], (double)-uy);
+  atomicAdd(&s_F[3 * a + 2], (double)-uz);
 }
 
-template <typename T, int W, int GNZ, bool Z16, bool FG>
-__global__ __launch_bounds__(256) void k_desc_bwd(int N, const int *__restrict__ species,
+// Doubles of the accumulators' region: T and F of W waves, or g if larger.
+template <typename T, int W>
+__host__ __device__ constexpr int bwd_acc_doubles(const Lds &L) {
+  return 4 * W * L.KP * 8 >= L.Dp * (int)sizeof(T) ? 4 * W * L.KP : L.Dp * (int)sizeof(T) / 8;
+}
+
+// FORM: 0 the generic form; for grid tables of NZ zetas NZ, NZ + 10 or NZ + 20
+// with ES = 1, 2 or 0: at most 4 ES etas, whose g stays in registers
+// (ang_bwd_grid), or any number, read from LDS records.
+constexpr int bwd_form(int nz, int es) { return nz == 0 ? 0 : nz + (es == 1 ? 0 : es == 2 ? 10 : 20); }
+constexpr int form_sets(int form) { return form == 0 || form >= 20 ? 0 : form >= 10 ? 2 : 1; }
+//
+// LDS bounds the workgroups in flight (96 bytes per neighbour in FP64, 64 in
+// FP32, beside it), so g shares its place with the accumulators, which start
+// once it has gone into registers and records.
+//
+// Measured, one wave per atom: 67,647 atoms of 45 to 95 neighbours (D = 128,
+// four etas) FP64 1710 -> 1280 us, mixed 781 -> 673 us; 4096 atoms FP64 152 ->
+// 118 us, mixed 78 -> 64 us; 32,768 atoms of 91 neighbours (D = 256, eight
+// etas) mixed 944 -> 794 us.  Of the mixed 694 us before the shared place the
+// triplets took about 455 (their instructions issue for about 400 of them), the
+// radial lines 85, the neighbours' tables 72, the contraction's finish 61.
+//
+// The bound of two waves per SIMD (256 registers) keeps the matrix results in
+// ordinary vector registers; without it they would be copied from the
+// accumulation registers, 16 more instructions per triplet.
+template <typename T, int W, int FORM, bool Z16, bool FG>
+__global__ __launch_bounds__(W > 4 ? 64 * W : 256, 2) void k_desc_bwd(int N, const int *__restrict__ species,
                                                   const double *__restrict__ wz, NeighborBufs nb, TripletBufs tb,
                                                   SFDev sf, Lds L, GradSrc gs, double *__restrict__ slot_f,
                                                   double *__restrict__ atom_vir) {
+  constexpr int GNZ = FORM % 10, ES = form_sets(FORM);
   extern __shared__ __align__(16) unsigned char smem[];
   if ((int)blockIdx.x >= N) return;  // one workgroup per atom of [atom0, atom0 + N)
   const int i = L.atom0 + blockIdx.x;
-  const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
+  const int tid = threadIdx.x, wv = wave_index(), lane = tid & 63;
   const int KP = L.KP, Dp = L.Dp, G = L.G;
   // per-wave accumulators in FP64 for both precisions (LDS FP64 atomics are
   // also the faster ones here), summed in wave order at the end: deterministic
   double *s_vir = (double *)smem;  // [W * 6]
   double *s_T = s_vir + 6 * W;     // [W][KP]
   double *s_F = s_T + W * KP;      // [W][3 KP]
-  T *s_d = (T *)(s_F + 3 * W * KP);
+  T *s_g = (T *)s_T;               // [Dp] g, until the accumulators start
+  T *s_d = (T *)(s_T + bwd_acc_doubles<T, W>(L));
   T *s_rw = s_d + 4 * KP;    // [KP] pairs (1 / r, species weight)
   // [G][KP] pairs (fc, dfc/dr) per cutoff group, in LDS or (FG) in the
   // atom's row of the global buffer
   T *s_fd = FG ? (T *)nb.fc_scratch + (size_t)i * 2 * G * KP : s_rw + 2 * KP;
-  T *s_g = FG ? s_rw + 2 * KP : s_fd + 2 * G * KP;
-  // generic form: per angular line, g of the plain and of the weighted
-  // feature; s_gW starts on a 4-value boundary (n_ang <= Dp / 2)
-  T *s_gA = s_g + Dp;
-  T *s_gW = s_gA + ((sf.n_ang + 3) & ~3);
-  // grid form: one record per eta, [g plain (2 NZ) | g weighted (2 NZ) | eta |
-  // exp coefficient | pad], so that a pass reads its eta's values from one
-  // base address; 16-byte aligned records (every region above has a multiple
-  // of 4 values), at most 2 Dp values (n_eta <= Dp / (4 NZ))
+  // radial lines: records (g plain, g weighted, exp coefficient, rs)
+  T *s_rr = FG ? s_rw + 2 * KP : s_fd + 2 * G * KP;
+  // generic form: per angular line, g of the plain and of the weighted feature
+  T *s_gA = s_rr + 4 * sf.n_rad;
+  T *s_gW = s_gA + sf.n_ang;
+  // grid form without registers (ES = 0): one record per eta, [g plain (2 NZ) |
+  // g weighted (2 NZ) | eta | exp coefficient | pad], so that a pass reads its
+  // eta's values from one base address; 16-byte aligned records (every region
+  // above has a multiple of 4 values).  An eta's record has at most 8 NZ values
+  // for its 2 NZ lines, so the radial and the angular regions together hold
+  // at most 4 (n_rad + n_ang) <= 2 Dp values.
   constexpr int RS = EtaRec<GNZ>::RS;
-  T *s_er = s_g + Dp;
+  static_assert(RS <= 8 * GNZ, "radial and eta records within 2 Dp values");
+  T *s_er = s_gA;
 
   const int start = i * nb.kcap;
   const int K = nb.nb_count[i];
@@ -953,24 +1224,8 @@ __global__ __launch_bounds__(256) void k_desc_bwd(int N, const int *__restrict__
     if (tid == 0) atomicAdd(&nb.total[3], 1);
     return;
   }
-  for (int a = tid; a < K; a += 64 * W) {
-    const double *dd = nb.nb_d + 4 * (size_t)(start + a);
-    const double r = dd[3];
-    s_d[4 * a] = (T)dd[0];
-    s_d[4 * a + 1] = (T)dd[1];
-    s_d[4 * a + 2] = (T)dd[2];
-    s_d[4 * a + 3] = (T)r;
-    s_rw[2 * a] = (T)(1.0 / r);
-    s_rw[2 * a + 1] = (T)slot_weight(nb, wz, species, start + a);
-    for (int g = 0; g < sf.n_groups; ++g) {
-      const double rc = sf.group_rc[g];
-      const bool in = r <= rc;
-      s_fd[2 * (g * KP + a)] = in ? (T)(0.5 * (cos(kPi * r / rc) + 1.0)) : T(0);
-      s_fd[2 * (g * KP + a) + 1] = in ? (T)(0.5 * (-sin(kPi * r / rc)) * (kPi / rc)) : T(0);
-    }
-  }
-  for (int k = tid; k < 4 * W * KP; k += 64 * W) s_T[k] = 0.0;  // s_T and s_F
-  if (GNZ > 0)
+  stage_neighbours<T, true>(nb, wz, species, sf, start, K, KP, s_d, s_rw, s_fd, tid, 64 * W);
+  if (GNZ > 0 && ES == 0)
     for (int h = tid; h < sf.n_eta; h += 64 * W) {
       s_er[h * RS + 4 * GNZ] = (T)sf.ang_eta[h * 2 * GNZ];
       s_er[h * RS + 4 * GNZ + 1] = eta_coef<T>((T)sf.ang_eta[h * 2 * GNZ]);
@@ -980,27 +1235,50 @@ __global__ __launch_bounds__(256) void k_desc_bwd(int N, const int *__restrict__
     // the contraction's finish for this atom (same order as k_gpr_finish)
     const double E = split_sum(gs.splits, [&](int sp) { return gs.Epart[(size_t)sp * gs.Np + i]; });
     if (tid == 0) gs.eatom[i] = E;
-    for (int d = tid; d < Dp; d += 64 * W) {
-      const double G =
-          gs.Gpart ? split_sum(gs.splits, [&](int sp) { return gs.Gpart[((size_t)sp * gs.Np + i) * Dp + d]; })
-                   : split_sum(gs.splits,
-                               [&](int sp) { return (double)gs.Gpart32[((size_t)sp * gs.Np + i) * Dp + d]; });
-      const double xt = gs.xt64 ? gs.xt64[row + d] : (double)gs.xt32[row + d];
-      const double g = -(xt * E - G) * gs.theta_inv[d];
-      if (gs.g64_out) {
-        gs.g64_out[row + d] = g;
-        s_g[d] = (T)g;
+    // two features per thread: Dp is a multiple of 32, rows are 16-byte aligned
+    for (int d = 2 * tid; d < Dp; d += 128 * W) {
+      double G0, G1;
+      const size_t at = (size_t)i * Dp + d, step = (size_t)gs.Np * Dp;
+      if (gs.Gpart) {
+        auto part = [&](int sp) { return *(const double2 *)(gs.Gpart + sp * step + at); };
+        split_sum2(gs.splits, part, G0, G1);
       } else {
-        const float gf = (float)g;
-        gs.g32_out[row + d] = gf;
-        s_g[d] = (T)gf;
+        auto part = [&](int sp) { return *(const float2 *)(gs.Gpart32 + sp * step + at); };
+        split_sum2(gs.splits, part, G0, G1);
+      }
+      double x0, x1;
+      if (gs.xt64) {
+        const double2 x = *(const double2 *)(gs.xt64 + at);
+        x0 = x.x, x1 = x.y;
+      } else {
+        const float2 x = *(const float2 *)(gs.xt32 + at);
+        x0 = (double)x.x, x1 = (double)x.y;
+      }
+      const double2 ti = *(const double2 *)(gs.theta_inv + d);
+      const double g0 = -(x0 * E - G0) * ti.x, g1 = -(x1 * E - G1) * ti.y;
+      if (gs.g64_out) {
+        *(double2 *)(gs.g64_out + at) = make_double2(g0, g1);
+        s_g[d] = (T)g0;
+        s_g[d + 1] = (T)g1;
+      } else {
+        const float f0 = (float)g0, f1 = (float)g1;
+        *(float2 *)(gs.g32_out + at) = make_float2(f0, f1);
+        s_g[d] = (T)f0;
+        s_g[d + 1] = (T)f1;
       }
     }
   } else {
     for (int d = tid; d < Dp; d += 64 * W) s_g[d] = gs.g64 ? (T)gs.g64[row + d] : (T)gs.g32[row + d];
   }
   __syncthreads();
-  for (int s = tid; s < sf.n_ang; s += 64 * W) {
+  for (int s = tid; s < sf.n_rad; s += 64 * W) {
+    const int f = sf.rad_feat[s];
+    s_rr[4 * s] = s_g[f];
+    s_rr[4 * s + 1] = s_g[f + sf.nsf];
+    s_rr[4 * s + 2] = eta_coef<T>(rad_table<T>(sf.rad_a, sf.rad_a32, s));
+    s_rr[4 * s + 3] = rad_table<T>(sf.rad_rs, sf.rad_rs32, s);
+  }
+  for (int s = tid; s < (ES > 0 ? 0 : sf.n_ang); s += 64 * W) {
     const int f = sf.ang_feat[s];
     if constexpr (GNZ > 0) {
       const int h = s / (2 * GNZ), k = s - h * 2 * GNZ;
@@ -1011,29 +1289,65 @@ __global__ __launch_bounds__(256) void k_desc_bwd(int N, const int *__restrict__
       s_gW[s] = s_g[f + sf.nsf];
     }
   }
-  __syncthreads();
+  // registers of the grid form: g over the lanes, the etas and their
+  // exponential coefficients (uniform; 0 past the last eta)
+  EtaRegs<T, ES> er;
+  T ceta[4 * ES + 1], eta[4 * ES + 1];
+  if constexpr (ES > 0) {
+#pragma unroll
+    for (int h = 0; h < 4 * ES; ++h) {
+      eta[h] = h < sf.n_eta ? (T)sf.ang_eta[h * 2 * GNZ] : T(0);
+      ceta[h] = eta_coef<T>(eta[h]);
+    }
+    if constexpr (sizeof(T) == 4) {
+#pragma unroll
+      for (int u = 0; u < ES; ++u) er.set[u] = load_eta_set<GNZ>(sf, s_g, u, lane);
+    } else {
+#pragma unroll
+      for (int h = 0; h < 4; ++h) {
+        const int z = lane & 15;
+        const bool live = h < sf.n_eta && z < 2 * GNZ;
+        const int f = live ? sf.ang_feat[h * 2 * GNZ + z] : 0;
+        er.ga[h] = live ? s_g[f] : 0.0;
+        er.gw[h] = live ? s_g[f + sf.nsf] : 0.0;
+      }
+    }
+  }
+  __syncthreads();  // g is consumed: its place becomes the accumulators
+  // this wave's vector accumulators (its s_T row is written by the radial part)
+  for (int k = lane; k < 3 * K; k += 64) s_F[3 * wv * KP + k] = 0.0;
 
-  // radial: one neighbour per thread
-  for (int a = tid; a < K; a += 64 * W) {
+  // radial: the lines split over the waves, 64 neighbours at a time; the last
+  // R < 64 of a longer list (half of the atoms of a usual cell have one) take
+  // 2^lg lanes per neighbour, each with a share of the lines
+  typedef typename Pair<T>::type P2;
+  for (int a0 = 0; a0 < K; a0 += 64) {
+    const int R = K - a0;
+    const int lg = R > 32 ? 0 : R > 16 ? 1 : R > 8 ? 2 : R > 4 ? 3 : 4;
+    const int part = lane & ((1 << lg) - 1), a = min(a0 + (lane >> lg), K - 1);
     const T r = s_d[4 * a + 3], w = s_rw[2 * a + 1];
     T acc = 0;
-    for (int s = 0; s < sf.n_rad; ++s) {
-      const int f = sf.rad_feat[s];
-      const int g = sf.rad_group[s];
-      const T A = rad_table<T>(sf.rad_a, sf.rad_a32, s);
-      const T dr = r - rad_table<T>(sf.rad_rs, sf.rad_rs32, s);
-      const T geff = s_g[f] + w * s_g[f + sf.nsf];
-      acc += geff * Math<T>::ex(-A * dr * dr) * (T(-2) * A * dr * s_fd[2 * (g * KP + a)] + s_fd[2 * (g * KP + a) + 1]);
+    int g = sf.rad_g;  // the cutoff group of every radial line, or -1
+    P2 f = ((const P2 *)s_fd)[max(g, 0) * KP + a];  // (fc, dfc)
+    for (int s = (wv << lg) + part; s < sf.n_rad; s += W << lg) {
+      const Quad<T> q = ((const Quad<T> *)s_rr)[s];  // g, g weighted, c, rs
+      if (sf.rad_g < 0 && sf.rad_group[s] != g) {
+        g = sf.rad_group[s];
+        f = ((const P2 *)s_fd)[g * KP + a];
+      }
+      // d/dr [exp(-A (r - rs)^2) fc], with c = -A log2(e) in FP32
+      const T dr = r - q.v[3], x = q.v[2] * dr;
+      acc += (q.v[0] + w * q.v[1]) * (exp_coef(x, dr) * (x * (slope_factor<T>() * f.x) + f.y));
     }
-    s_T[a] = (double)acc;  // wave 0's row
+    for (int o = 1; o < 1 << lg; o <<= 1) acc += __shfl_xor(acc, o, 64);
+    if (part == 0 && a0 + (lane >> lg) < K) s_T[wv * KP + a] = (double)acc;
   }
   __syncthreads();
-
 
   if (sf.n_ang > 0) {
     const uint32_t *tl = tb.list + (size_t)i * tb.tcap;
     const int nt = tb.count[i];
-    const T rcA = (T)sf.group_rc[sf.g_ang], pirc = (T)(kPi / sf.group_rc[sf.g_ang]);
+    const T rcA = (T)sf.group_rc[sf.g_ang], pirc = (T)sf.group_pirc[sf.g_ang];
     constexpr int ST = 64 * W;
     uint32_t qc[4], qn[4];
     load_q4(tl, nt, 64 * wv + lane, ST, qc);
@@ -1041,11 +1355,12 @@ __global__ __launch_bounds__(256) void k_desc_bwd(int N, const int *__restrict__
       load_q4(tl, nt, t0 + 4 * ST + lane, ST, qn);
 #pragma unroll 1
       for (int u = 0; u < 4; ++u) {
+        if (t0 + u * ST >= nt) break;
         const bool act = t0 + u * ST + lane < nt;
         const uint32_t q = pop_q4(qc);
         if constexpr (GNZ > 0)
-          ang_bwd_grid<T, GNZ, Z16>(q, act, sf, s_d, s_rw, s_fd, s_er, KP, rcA, pirc, s_T + wv * KP,
-                                    s_F + 3 * wv * KP);
+          ang_bwd_grid<T, GNZ, Z16, ES>(q, act, sf, s_d, s_rw, s_fd, s_er, er, ceta, eta, KP, rcA, pirc,
+                                        s_T + wv * KP, s_F + 3 * wv * KP);
         else
           ang_bwd_term<T>(q, act, sf, s_d, s_rw, s_fd, s_gA, s_gW, KP, s_T + wv * KP, s_F + 3 * wv * KP);
       }
@@ -1092,11 +1407,8 @@ __global__ __launch_bounds__(256) void k_desc_bwd(int N, const int *__restrict__
     vir[4] += sc * dy * dz + Fy * dz;
     vir[5] += sc * dx * dz + Fx * dz;
   }
-#pragma unroll
-  for (int c = 0; c < 6; ++c) {
-    const double v = wave_sum(vir[c]);
-    if (lane == 0) s_vir[6 * wv + c] = v;
-  }
+  const double vt = wave_totals<double, 6>(vir, lane);
+  if (lane < 6) s_vir[6 * wv + lane] = vt;
   __syncthreads();
   if (tid < 6) {
     double v = 0.0;
@@ -1109,13 +1421,21 @@ __global__ __launch_bounds__(256) void k_desc_bwd(int N, const int *__restrict__
 // LDS bytes of each kernel's layout; FG: the cutoff tables in global memory.
 template <typename T, int NCH, int W, bool FG>
 size_t fwd_lds(const Lds &L) {
-  return W * sizeof(double) + (size_t)(4 * L.KP + L.KP + (FG ? 0 : L.G * L.KP) + L.Dp + W * 2 * NCH) * sizeof(T);
+  return ((W + 1) & ~1) * sizeof(double) +
+         (size_t)(6 * L.KP + (FG ? 0 : L.G * L.KP) + L.Dp + W * 2 * NCH) * sizeof(T);
 }
 
+// REGS: the register form of the grid backward, without angular g records.
 template <typename T, int W, bool FG>
-size_t bwd_lds(const Lds &L) {
-  return (6 * W + 4 * W * (size_t)L.KP) * sizeof(double) +
-         (size_t)(6 * L.KP + (FG ? 0 : 2 * L.G * L.KP) + 3 * L.Dp) * sizeof(T);
+size_t bwd_lds(const Lds &L, bool regs) {
+  return (6 * W + (size_t)bwd_acc_doubles<T, W>(L)) * sizeof(double) +
+         (size_t)(6 * L.KP + (FG ? 0 : 2 * L.G * L.KP) + (regs ? 4 * L.n_rad : 2 * L.Dp)) * sizeof(T);
+}
+
+// The layout that sets the longest accepted list: every other one is smaller.
+template <typename T>
+size_t list_limit_lds(const Lds &L) {
+  return (6 + 4 * (size_t)L.KP) * sizeof(double) + (size_t)(6 * L.KP + 3 * L.Dp) * sizeof(T);
 }
 
 template <typename T, int NZ, int W, bool FG>
@@ -1218,15 +1538,34 @@ bool zeta_1_2_4_16(const SFDev &sf) {
   return sf.nz == 4 && sf.zlog[0] == 0 && sf.zlog[1] == 1 && sf.zlog[2] == 2 && sf.zlog[3] == 4;
 }
 
+// Whether the backward keeps g in registers: a grid of at most four etas, or
+// in FP32 eight.
+template <typename T>
+bool bwd_regs(const SFDev &sf) {
+  return sf.grid && sf.n_eta <= (sizeof(T) == 4 ? 8 : 4);
+}
+
+template <typename T, int W, int GNZ, bool Z16, bool FG, int ES>
+hipError_t bwd_launch_as(hipStream_t s, int N, const int *species, const double *wz, const NeighborBufs &nb,
+                      const TripletBufs &tb, const SFDev &sf, Lds L, const GradSrc &gs, double *slot_f,
+                      double *atom_vir) {
+  const size_t lds = bwd_lds<T, W, FG>(L, ES > 0);
+  const hipError_t e = allow_lds((const void *)k_desc_bwd<T, W, bwd_form(GNZ, ES), Z16, FG>, lds);
+  if (e != hipSuccess) return e;
+  k_desc_bwd<T, W, bwd_form(GNZ, ES), Z16, FG><<<N, 64 * W, lds, s>>>(N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
+  return hipGetLastError();
+}
+
 template <typename T, int W, int GNZ, bool Z16, bool FG>
 hipError_t bwd_launch(hipStream_t s, int N, const int *species, const double *wz, const NeighborBufs &nb,
                       const TripletBufs &tb, const SFDev &sf, Lds L, const GradSrc &gs, double *slot_f,
                       double *atom_vir) {
-  const size_t lds = bwd_lds<T, W, FG>(L);
-  const hipError_t e = allow_lds((const void *)k_desc_bwd<T, W, GNZ, Z16, FG>, lds);
-  if (e != hipSuccess) return e;
-  k_desc_bwd<T, W, GNZ, Z16, FG><<<N, 64 * W, lds, s>>>(N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
-  return hipGetLastError();
+  if constexpr (GNZ > 0) {
+    if (sf.n_eta <= 4) return bwd_launch_as<T, W, GNZ, Z16, FG, 1>(s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
+    if constexpr (sizeof(T) == 4)
+      if (sf.n_eta <= 8) return bwd_launch_as<T, W, GNZ, Z16, FG, 2>(s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
+  }
+  return bwd_launch_as<T, W, GNZ, Z16, FG, 0>(s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
 }
 
 template <typename T, int W, bool FG>
@@ -1296,7 +1635,7 @@ hipError_t fwd_grid(int waves, hipStream_t s, int N, const int *species, const d
 template <typename T>
 bool needs_global_tables(const SFDev &sf, const Lds &L) {
   const size_t lim = lds_limit();
-  if (bwd_lds<T, 1, false>(L) > lim) return true;
+  if (bwd_lds<T, 1, false>(L, bwd_regs<T>(sf)) > lim) return true;
   if (!sf.grid) return fwd_lds<T, 16, 1, false>(L) > lim;
   return fwd_grid_lds<T, 5, 1, false>(L) > lim;  // the widest grid layout
 }
@@ -1305,7 +1644,7 @@ bool needs_global_tables(const SFDev &sf, const Lds &L) {
 template <typename T>
 bool fits(const SFDev &sf, const Lds &L) {
   const size_t lim = lds_limit();
-  if (bwd_lds<T, 1, true>(L) > lim) return false;
+  if (list_limit_lds<T>(L) > lim) return false;
   if (!sf.grid) return fwd_lds<T, 16, 1, true>(L) <= lim;
   return fwd_grid_lds<T, 5, 1, true>(L) <= lim;
 }
@@ -1317,9 +1656,10 @@ hipError_t bwd_fit(int waves, hipStream_t s, int N, const int *species, const do
   int W;
   bool fg;
   auto bytes = [&](int w, bool g) {
-    if (w == 4) return bwd_lds<T, 4, false>(L);
-    if (w == 2) return bwd_lds<T, 2, false>(L);
-    return g ? bwd_lds<T, 1, true>(L) : bwd_lds<T, 1, false>(L);
+    const bool regs = bwd_regs<T>(sf);
+    if (w == 4) return bwd_lds<T, 4, false>(L, regs);
+    if (w == 2) return bwd_lds<T, 2, false>(L, regs);
+    return g ? bwd_lds<T, 1, true>(L, regs) : bwd_lds<T, 1, false>(L, regs);
   };
   if (!pick_shape(waves, 4, bytes, W, fg) || (fg && !nb.fc_scratch)) return hipErrorInvalidValue;
   if (fg) return bwd_grid<T, 1, true>(s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
@@ -1337,7 +1677,7 @@ int max_neighbors_for_lds(bool fp64, const SFDev &sf, int Dp) {
   const int G = sf.n_groups > 0 ? sf.n_groups : 1;
   int kp = kMaxNeighbors;
   for (; kp > 8; kp -= 8) {
-    const Lds L{kp, G, Dp, 0};
+    const Lds L{kp, G, Dp, 0, sf.n_rad};
     if (fp64 ? fits<double>(sf, L) : fits<float>(sf, L)) break;
   }
   return kp;
@@ -1345,7 +1685,7 @@ int max_neighbors_for_lds(bool fp64, const SFDev &sf, int Dp) {
 
 size_t desc_table_scratch_bytes(bool fp64, const SFDev &sf, int Dp, int KP, int N) {
   const int G = sf.n_groups > 0 ? sf.n_groups : 1;
-  const Lds L{KP, G, Dp, 0};
+  const Lds L{KP, G, Dp, 0, sf.n_rad};
   if (!(fp64 ? needs_global_tables<double>(sf, L) : needs_global_tables<float>(sf, L))) return 0;
   return (size_t)N * 2 * G * KP * (fp64 ? sizeof(double) : sizeof(float));
 }
@@ -1354,7 +1694,7 @@ hipError_t launch_descriptors_fwd(hipStream_t s, bool fp64, int N, const int *sp
                                   const NeighborBufs &nb, const TripletBufs &tb, const SFDev &sf,
                                   const double *theta_inv, const double *mu, int split_mode, DescOut out, int chunk,
                                   int waves, int KP, int atom0) {
-  Lds L{KP, sf.n_groups > 0 ? sf.n_groups : 1, out.Dp, atom0};
+  Lds L{KP, sf.n_groups > 0 ? sf.n_groups : 1, out.Dp, atom0, sf.n_rad};
   if (N <= 0) return hipSuccess;
   if (sf.grid) {
     if (fp64) return fwd_grid<double>(waves, s, N, species, wz, nb, tb, sf, L, theta_inv, mu, split_mode, out);
@@ -1372,7 +1712,7 @@ hipError_t launch_descriptors_bwd(hipStream_t s, bool fp64, int N, const int *sp
                                   const NeighborBufs &nb, const TripletBufs &tb, const SFDev &sf, int Dp,
                                   const GradSrc &gs, double *slot_f, double *atom_vir, int waves, int KP,
                                   int atom0) {
-  Lds L{KP, sf.n_groups > 0 ? sf.n_groups : 1, Dp, atom0};
+  Lds L{KP, sf.n_groups > 0 ? sf.n_groups : 1, Dp, atom0, sf.n_rad};
   if (N <= 0) return hipSuccess;
   // the LDS layout's 16-byte reads of g need KP (slots per atom) a multiple of 4
   if (KP % 4 != 0) return hipErrorInvalidValue;

@@ -5,6 +5,7 @@
 
 #include <cstdint>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 struct gapx_mlp;
@@ -43,6 +44,7 @@ struct SFDev {
   // cutoff group and the sorted lines are eta x (lambda = +1, -1) x zeta with
   // the same zeta list, zeta in {1, 2, 4, 8, 16}): line s = h * 2 nz + li * nz + k.
   int grid, n_eta, nz, g_ang;
+  int rad_g;               // cutoff group of every radial line, -1 when they differ
   int zlog[5];             // log2 zeta_k
   double zeta_k[5], pref_k[5];
   const double *rad_a, *rad_rs;
@@ -50,7 +52,7 @@ struct SFDev {
   const int *rad_group, *rad_feat;
   const double *ang_eta, *ang_lam, *ang_pref, *ang_zeta_real;
   const int *ang_zeta, *ang_group, *ang_feat;
-  const double *group_rc;
+  const double *group_rc, *group_pirc;  // cutoff of each group, kPi / cutoff
 };
 
 struct Model {
@@ -223,20 +225,34 @@ hipError_t launch_descriptors_fwd(hipStream_t s, bool fp64, int N, const int *sp
 // finished from the contraction's split partials inside the backward kernel
 // (splits > 0): E_i = sum_s Epart[s][i] and g = -(xt E - sum_s G[s][i]) theta_inv,
 // summed in split order; E_i goes to eatom and g to g64/g32 as well.
-// sum_{sp < n} load(sp) in ascending sp, with the loads issued eight at a
-// time (a plain loop's accumulation makes every load wait for the one
-// before it).  n >= 0; load is called with indices in [0, n) only.
+// sum_{sp < n} load(sp) in ascending sp (pairs: v.x and v.y), with the loads
+// issued eight at a time and then four, two and one (a plain loop's
+// accumulation makes every load wait for the one before it).  n >= 0.
+template <typename F>
+__device__ __forceinline__ void split_sum2(int n, F load, double &s0, double &s1) {
+  s0 = s1 = 0.0;
+  int at = 0;
+  auto batch = [&](auto count) {
+    constexpr int C = decltype(count)::value;
+    decltype(load(0)) v[C];
+#pragma unroll
+    for (int u = 0; u < C; ++u) v[u] = load(at + u);
+#pragma unroll
+    for (int u = 0; u < C; ++u) {
+      s0 += (double)v[u].x;
+      s1 += (double)v[u].y;
+    }
+    at += C;
+  };
+  while (at + 8 <= n) batch(std::integral_constant<int, 8>{});
+  if (n & 4) batch(std::integral_constant<int, 4>{});
+  if (n & 2) batch(std::integral_constant<int, 2>{});
+  if (n & 1) batch(std::integral_constant<int, 1>{});
+}
 template <typename F>
 __device__ __forceinline__ double split_sum(int n, F load) {
-  double s = 0.0;
-  for (int s0 = 0; s0 < n; s0 += 8) {
-    double v[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v[u] = load(min(s0 + u, n - 1));
-#pragma unroll
-    for (int u = 0; u < 8; ++u)
-      if (s0 + u < n) s += v[u];
-  }
+  double s, unused;
+  split_sum2(n, [&](int sp) { return make_double2(load(sp), 0.0); }, s, unused);
   return s;
 }
 
