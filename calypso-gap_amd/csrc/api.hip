@@ -427,6 +427,10 @@ struct Ctx {
   bool ran = false;
   int chunk = 0;  // lines per forward pass of the generic kernels (0: 16)
   Tuning tune[2];  // launch shapes for FP64 [0] and mixed [1] runs
+  // shapes given by the caller, the environment or the autotuner: loads keep
+  // them; otherwise every load sets them by its size (default_tuning)
+  bool tune_given[2] = {false, false};
+  bool waves_fwd_given = false, waves_bwd_given = false;  // by the environment
   Mlp *mlp = nullptr;  // set while the last run used the surrogate
   bool md_ready = false;  // md_p holds the momenta of the last MD run
   unsigned long long bins_clean = ~0ULL;  // allocation generations of bin_count/bin_ticket last cleared
@@ -584,6 +588,83 @@ static int struct_params(Ctx &c) {
   return GAPX_OK;
 }
 
+// Splits of the sparse points for a contraction of `tiles` row tiles, least
+// in an estimate of its time in chunks (of 64 or 32 points); returns that time.
+// The chip holds `slots` workgroups.  `over`: a workgroup's start and end,
+// `part`: the later reads of one split's partial sums.
+// The mixed kernel waits for its operands rather than for the matrix cores, so
+// a round that is started costs a whole one.  The FP64 kernel (soft) is bound
+// by its matrix products: workgroups past the first round share what is left,
+// and only about 0.45 of the last workgroup's length stays exposed.
+static double best_splits(int tiles, int slots, int chunks, double over, double part, bool soft, int *splits) {
+  double best = 1e300;
+  for (int want = 1; want <= std::min(chunks, 64); ++want) {
+    const int per = (chunks + want - 1) / want, s = (chunks + per - 1) / per;
+    const double rounds = (double)tiles * s / slots;
+    double cost;
+    if (soft)
+      cost = (rounds <= 1.0 ? per : (double)tiles * chunks / slots + 0.45 * per) + over * std::max(1.0, rounds);
+    else
+      cost = std::ceil(rounds) * (per + over);
+    cost += s * part;
+    if (cost < best * 0.999) {
+      best = cost;
+      *splits = s;
+    }
+  }
+  return best;
+}
+
+// Launch shapes by the batch's size, for contexts whose caller gave none.
+// The contraction's split used to aim at 512 workgroups whatever the tiles:
+// 67,647 atoms gave 1058 FP64 workgroups for the chip's 512 places and 529
+// mixed ones (a second round for 17 of them).  Measured there, us by splits:
+// FP64 1: 2700, 3: 2440, 4: 2365, 6: 2303; mixed 1: 489, 2: 403, 3: 381,
+// 4: 373, 6: 364, 8: 380, the backward then 3 (mixed) or 6 us (FP64) longer
+// per split.  At 4096 atoms the rule keeps one full round (FP64 8 splits
+// 157 us, 12: 176, 16: 167; mixed 36 for 64- and 128-row tiles); at 197 atoms
+// 64-row tiles give twice the workgroups (11.3 against 13.9 us).  A chunk of
+// 64 points takes a workgroup about 16 us in FP64 and 3.9 us mixed (128 rows,
+// D = 128; 64 rows 0.71 of it), its start and end 0.2 FP64 and three mixed ones.
+static void default_tuning(Ctx &c) {
+  const Model &m = *c.m;
+  for (int p = 0; p < 2; ++p) {
+    if (c.tune_given[p]) continue;
+    Tuning &t = c.tune[p];
+    const bool fp64 = p == 0, c64 = fp64 || m.mixed_f64, grid = m.sfd.grid != 0;
+    // two overlapped halves pay only where the contraction leaves registers
+    // free (replayed 67,647 atoms: mixed 1729 against 1754 us, FP64 5055
+    // against 5100 but eager 5190 against 5100; 32,768 atoms with D = 256,
+    // one workgroup a CU, 2341 against 2323, eager 2460 against 2300)
+    t.halves = (!c64 && m.Dp <= 128) ? 1 : 0;
+    if (!c.waves_fwd_given) t.waves_fwd = waves_within(c.N, fwd_wave_cap(fp64), 1);
+    if (!c.waves_bwd_given) t.waves_bwd = waves_within(c.N, bwd_wave_cap(fp64, grid), !grid ? 4 : 1);
+    const int pts = gpr_points_per_chunk(m.Dp), chunks = m.Mp / pts;
+    const double scale = m.Dp / 128.0 * pts / 64.0;
+    const double part_us = (double)c.Np * m.Dp * (c64 ? 8 : 4) / 1e7;
+    if (c64) {
+      const int tiles = c.Np / 64, slots = m.Dp <= 160 ? 512 : 256;
+      int s = 1;
+      best_splits(tiles, slots, chunks, 0.2, part_us / (16.0 * scale), true, &s);
+      t.gpr_blocks = std::min(tiles * s, 1 << 20);
+      continue;
+    }
+    double best = 1e300;
+    for (int rows : {128, 64}) {
+      if (rows == 64 && m.Dp > 128) continue;  // 128-row tiles only
+      const int tiles = c.Np / rows;
+      const double chunk_us = 3.9 * scale * (rows == 64 ? 0.71 : 1.0);
+      int s = 1;
+      const double us = chunk_us * best_splits(tiles, m.Dp <= 128 ? 512 : 256, chunks, 3.0, part_us / chunk_us, false, &s);
+      if (us < best) {
+        best = us;
+        t.gpr_rows = rows;
+        t.gpr_blocks = std::min(tiles * s, 1 << 20);
+      }
+    }
+  }
+}
+
 // Initial slots per atom from the densest structure of the batch.
 static int initial_tcap(const Ctx &c) {
   // pairs within the angular cutoff: about (15/32) K (K - 1) / 2 at uniform density
@@ -664,6 +745,7 @@ static int ctx_load_batch(Ctx &c, int nstruct, const int *natoms, const int *spe
   GAPX_HIP(hipStreamSynchronize(c.stream));
   c.kcap = initial_kcap(c);
   c.tcap = initial_tcap(c);
+  default_tuning(c);
   c.ran = false;
   c.md_ready = false;
   c.invalidate_graph();
@@ -1266,6 +1348,7 @@ static int ctx_autotune(Ctx &c, int flags, bool force) {
     auto it = g_tune_cache.find(key);
     if (it != g_tune_cache.end()) {
       c.tune[p] = it->second;
+      c.tune_given[p] = true;
       c.invalidate_graph();
       return GAPX_OK;
     }
@@ -1389,6 +1472,7 @@ static int ctx_autotune(Ctx &c, int flags, bool force) {
   c.use_graph = was_graph;
   c.invalidate_graph();
   if (rc) return rc;
+  c.tune_given[p] = true;
   std::lock_guard<std::mutex> lk(g_tune_mu);
   g_tune_cache[key] = t;
   return GAPX_OK;
@@ -1868,15 +1952,15 @@ static int ctx_create(Model *m, Ctx **out) {
     return fail(GAPX_ERR_NOMEM, "pinned host allocation failed");
   }
   std::memset(c->host_stats, 0, 8 * sizeof(int));
-  // Grid-form tables run fastest with one wavefront per atom (measured on the
-  // 4096-atom ternary cell, D = 128); the generic kernels with four.  The
-  // mixed contraction takes 128-row tiles (above D = 128 it has no other).
+  // Shapes before the first load (default_tuning sets them by the batch):
+  // one wavefront per atom for grid-form tables, four for generic ones;
+  // 128-row tiles for the mixed contraction.
   for (int p = 0; p < 2; ++p) {
     Tuning &t = c->tune[p];
     if (c->m->sfd.grid) t.waves_fwd = t.waves_bwd = 1;
     t.gpr_rows = p == 1 ? 128 : 64;
-    if (const char *w = std::getenv("GAPX_DESC_WAVES_FWD")) t.waves_fwd = std::atoi(w);
-    if (const char *w = std::getenv("GAPX_DESC_WAVES_BWD")) t.waves_bwd = std::atoi(w);
+    if (const char *w = std::getenv("GAPX_DESC_WAVES_FWD")) t.waves_fwd = std::atoi(w), c->waves_fwd_given = true;
+    if (const char *w = std::getenv("GAPX_DESC_WAVES_BWD")) t.waves_bwd = std::atoi(w), c->waves_bwd_given = true;
   }
   if (const char *ch = std::getenv("GAPX_DESC_CHUNK")) c->chunk = std::atoi(ch);
   *out = c;
@@ -2667,6 +2751,7 @@ int gapx_ctx_set_tuning(gapx_ctx *c, int flags, int waves_fwd, int waves_bwd, in
   t.gpr_rows = gpr_rows;
   t.gpr_blocks = gpr_blocks;
   t.halves = halves;
+  c->tune_given[(run_flags(*c->m, flags) & GAPX_MIXED) ? 1 : 0] = true;
   c->invalidate_graph();
   return GAPX_OK;
 }

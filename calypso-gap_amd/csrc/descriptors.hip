@@ -1493,7 +1493,7 @@ hipError_t allow_lds(const void *kernel, size_t bytes) {
 template <typename F>
 bool pick_shape(int waves, int wmax, F bytes, int &W, bool &fg) {
   fg = false;
-  for (int w = 4; w >= 2; w /= 2)
+  for (int w = 8; w >= 2; w /= 2)
     if (w <= wmax && waves >= w && bytes(w, false) <= kLdsBudget) {
       W = w;
       return true;
@@ -1522,14 +1522,16 @@ hipError_t fwd_waves(int waves, hipStream_t s, int N, const int *species, const 
   int W;
   bool fg;
   auto bytes = [&](int w, bool g) {
+    if (w == 8) return fwd_lds<T, NCH, 8, false>(L);
     if (w == 4) return fwd_lds<T, NCH, 4, false>(L);
     if (w == 2) return fwd_lds<T, NCH, 2, false>(L);
     return g ? fwd_lds<T, NCH, 1, true>(L) : fwd_lds<T, NCH, 1, false>(L);
   };
-  if (!pick_shape(waves, 4, bytes, W, fg) || (fg && !nb.fc_scratch)) return hipErrorInvalidValue;
+  if (!pick_shape(waves, 8, bytes, W, fg) || (fg && !nb.fc_scratch)) return hipErrorInvalidValue;
   if (fg) return fwd_launch<T, NCH, 1, true>(s, N, species, wz, nb, tb, sf, L, theta_inv, mu, split_mode, out);
   if (W == 1) return fwd_launch<T, NCH, 1, false>(s, N, species, wz, nb, tb, sf, L, theta_inv, mu, split_mode, out);
   if (W == 2) return fwd_launch<T, NCH, 2, false>(s, N, species, wz, nb, tb, sf, L, theta_inv, mu, split_mode, out);
+  if (W == 8) return fwd_launch<T, NCH, 8, false>(s, N, species, wz, nb, tb, sf, L, theta_inv, mu, split_mode, out);
   return fwd_launch<T, NCH, 4, false>(s, N, species, wz, nb, tb, sf, L, theta_inv, mu, split_mode, out);
 }
 
@@ -1604,11 +1606,15 @@ hipError_t fwd_grid_nz(int waves, hipStream_t s, int N, const int *species, cons
   int W;
   bool fg;
   auto bytes = [&](int w, bool g) {
+    if (w == 8) return fwd_grid_lds<T, NZ, 8, false>(L);
+    if (w == 4) return (size_t)-1;  // one, two or eight waves
     if (w == 2) return fwd_grid_lds<T, NZ, 2, false>(L);
     return g ? fwd_grid_lds<T, NZ, 1, true>(L) : fwd_grid_lds<T, NZ, 1, false>(L);
   };
-  if (!pick_shape(waves, 2, bytes, W, fg) || (fg && !nb.fc_scratch)) return hipErrorInvalidValue;
+  if (!pick_shape(waves, 8, bytes, W, fg) || (fg && !nb.fc_scratch)) return hipErrorInvalidValue;
   if (fg) return fwd_grid_launch<T, NZ, 1, Z, true>(s, N, species, wz, nb, tb, sf, L, theta_inv, mu, split_mode, out);
+  if (W == 8)
+    return fwd_grid_launch<T, NZ, 8, Z, false>(s, N, species, wz, nb, tb, sf, L, theta_inv, mu, split_mode, out);
   if (W == 2)
     return fwd_grid_launch<T, NZ, 2, Z, false>(s, N, species, wz, nb, tb, sf, L, theta_inv, mu, split_mode, out);
   return fwd_grid_launch<T, NZ, 1, Z, false>(s, N, species, wz, nb, tb, sf, L, theta_inv, mu, split_mode, out);
@@ -1657,12 +1663,14 @@ hipError_t bwd_fit(int waves, hipStream_t s, int N, const int *species, const do
   bool fg;
   auto bytes = [&](int w, bool g) {
     const bool regs = bwd_regs<T>(sf);
+    if (w == 8) return bwd_lds<T, 8, false>(L, regs);
     if (w == 4) return bwd_lds<T, 4, false>(L, regs);
     if (w == 2) return bwd_lds<T, 2, false>(L, regs);
     return g ? bwd_lds<T, 1, true>(L, regs) : bwd_lds<T, 1, false>(L, regs);
   };
-  if (!pick_shape(waves, 4, bytes, W, fg) || (fg && !nb.fc_scratch)) return hipErrorInvalidValue;
+  if (!pick_shape(waves, 8, bytes, W, fg) || (fg && !nb.fc_scratch)) return hipErrorInvalidValue;
   if (fg) return bwd_grid<T, 1, true>(s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
+  if (W == 8) return bwd_grid<T, 8, false>(s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
   if (W == 4) return bwd_grid<T, 4, false>(s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
   if (W == 2) return bwd_grid<T, 2, false>(s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
   return bwd_grid<T, 1, false>(s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
@@ -1696,6 +1704,7 @@ hipError_t launch_descriptors_fwd(hipStream_t s, bool fp64, int N, const int *sp
                                   int waves, int KP, int atom0) {
   Lds L{KP, sf.n_groups > 0 ? sf.n_groups : 1, out.Dp, atom0, sf.n_rad};
   if (N <= 0) return hipSuccess;
+  waves = widened(waves, N, fwd_wave_cap(fp64));
   if (sf.grid) {
     if (fp64) return fwd_grid<double>(waves, s, N, species, wz, nb, tb, sf, L, theta_inv, mu, split_mode, out);
     return fwd_grid<float>(waves, s, N, species, wz, nb, tb, sf, L, theta_inv, mu, split_mode, out);
@@ -1716,6 +1725,7 @@ hipError_t launch_descriptors_bwd(hipStream_t s, bool fp64, int N, const int *sp
   if (N <= 0) return hipSuccess;
   // the LDS layout's 16-byte reads of g need KP (slots per atom) a multiple of 4
   if (KP % 4 != 0) return hipErrorInvalidValue;
+  waves = widened(waves, N, bwd_wave_cap(fp64, sf.grid != 0));
   if (fp64) return bwd_fit<double>(waves, s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
   return bwd_fit<float>(waves, s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
 }

@@ -305,6 +305,27 @@ hipError_t launch_descriptors_bwd(hipStream_t s, bool fp64, int N, const int *sp
                                   const double *wz, const NeighborBufs &nb, const TripletBufs &tb,
                                   const SFDev &sf, int Dp, const GradSrc &gs,
                                   double *slot_f, double *atom_vir, int waves, int KP, int atom0 = 0);
+// Wavefronts per atom of the descriptor kernels for N atoms.  The chip holds a
+// few thousand of these waves (the FP64 kernels' registers and LDS fewer than
+// the FP32 ones'); up to there more waves per atom shorten each atom's serial
+// chain, past it they only repeat its preamble.  Measured on 14 A^3 per atom,
+// rcut 6 A, us for W = 1, 2, 4, 8 (the grid forward has no W = 4):
+//   FP64 forward   64 atoms 39 25 - 17,  512: 42 31 - 31,  1024: 45 36 - 54,  2048: 56 71 - 104
+//   FP64 backward  64: 50 34 26 24,  512: 56 45 34 47,  1024: 57 46 49 70,  2048: 73 78 74 120
+//   FP32 forward   64: 25 17 - 12,  512: 27 18 - 15,  1024: 28 22 - 25,  4096: 44 50 - 82
+//   FP32 backward  64: 33 25 22 20,  512: 38 31 27 25,  1024: 43 35 33 44,  67,647: 601 629 781 -
+//   generic FP64   64: 168 98 78 63 forward, 237 131 76 48 backward;
+//                  1024: 205 139 169 233, 273 173 158 178;  4096: 397 497 635 914, 793 541 462 685
+// so W is the largest with N W within these waves; the generic backward keeps
+// four whatever N.
+constexpr int fwd_wave_cap(bool fp64) { return fp64 ? 3072 : 4096; }
+constexpr int bwd_wave_cap(bool fp64, bool grid) { return !grid ? 5120 : fp64 ? 2560 : 4096; }
+// The launchers run four waves per atom as eight where N allows it.
+constexpr int widened(int waves, int N, int cap) { return waves == 4 && (long long)N * 8 <= cap ? 8 : waves; }
+constexpr int waves_within(int N, int cap, int least) {
+  return (long long)N * 4 <= cap ? 4 : (long long)N * 2 <= cap ? 2 > least ? 2 : least : least;
+}
+
 // Largest per-atom neighbour count the descriptor kernels take: within the
 // device's per-workgroup LDS (160 KB on gfx950) with the cutoff tables moved
 // to global memory where needed, and at most kMaxNeighbors.

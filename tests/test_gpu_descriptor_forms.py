@@ -90,3 +90,31 @@ def test_forms(form, vpa):
         x = ctx.results()
         assert np.abs(x["forces"] - r["forces"]).max() < 1e-4 * np.abs(r["forces"]).max()
         assert abs(x["energy"][0] - r["energy"][0]) < 1e-5 * np.abs(r["eatom"]).sum()
+
+
+def test_default_shapes_by_size(monkeypatch):
+    """Loads without given shapes take them from the batch's size: small
+    batches four to eight waves per atom and as many splits as there are
+    chunks, larger ones fewer.  Every size gives what one wave per atom and
+    one split give (FP64 sums in another order: 1e-12 of the largest value)."""
+    rng = np.random.default_rng(9)
+    first = synth.structure(8, 8 * 14.0, (1, 8, 22), rng)
+    m = gapx.Model.from_model(model_for(FORMS["eta4_zeta4"], first, rng))
+    seen = set()
+    for n in (2, 8, 65, 257, 321, 385, 641, 769, 1537, 3100):
+        s = synth.jittered_structures(1, n, n, 1.0 / 14.0, (1, 8, 22), n)[0]
+        ctx = gapx.Context(m)
+        ctx.load([s], 6.0)
+        t = ctx.tuning(gapx.GRAD)
+        seen.add((t["waves_fwd"], t["waves_bwd"]))
+        print(n, t, flush=True)
+        ctx.run(gapx.GRAD)
+        a = ctx.results()
+        ctx.set_tuning(gapx.GRAD, waves_fwd=1, waves_bwd=1, gpr_rows=64, gpr_blocks=1, halves=0)
+        ctx.run(gapx.GRAD)
+        b = ctx.results()
+        for k in ("energy", "forces", "stress", "eatom"):
+            assert np.abs(a[k] - b[k]).max() <= 1e-12 * max(1.0, np.abs(b[k]).max()), (n, k)
+        ctx.load([s], 6.0)  # given shapes stay across loads
+        assert ctx.tuning(gapx.GRAD)["gpr_blocks"] == 1
+    assert {w for w, _ in seen} == {1, 2, 4} and {w for _, w in seen} == {1, 2, 4}
