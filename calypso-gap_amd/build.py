@@ -6,6 +6,7 @@ Outputs (git-ignored, they travel with the tree):
     calypso-gap_amd/lib/libgapx.so              HIP kernels + C ABI (gfx950)
     calypso-gap_amd/lib/libgapx_fortran.so      Fortran host facade (FGAP_CALC, ...)
     calypso-gap_amd/libgap/libgap*.so           f2py module libgap.libgap
+    calypso-gap_amd/gapx/_pack*.so              structure packing of the Python binding
 
 Every HIP file is compiled for gfx950 only, with packed-FP32 instruction
 selection disabled.
@@ -100,6 +101,16 @@ def build_fortran():
     return mod
 
 
+def build_pack():
+    """gapx._pack: gathers lists of structures for the Python binding."""
+    import numpy
+    ext = sysconfig.get_config_var("EXT_SUFFIX") or ".so"
+    mod = os.path.join(HERE, "gapx", "_pack" + ext)
+    run(["gcc", "-O2", "-shared", "-fPIC", "-Wall", "-I" + sysconfig.get_paths()["include"],
+         "-I" + numpy.get_include(), os.path.join(HERE, "gapx", "_pack.c"), "-o", mod])
+    return mod
+
+
 def build_oracle():
     """The oracle: its C restatement always; the reference Fortran when it is mounted."""
     run(["make", "-s", "-C", os.path.join(ROOT, "oracle")])
@@ -110,6 +121,7 @@ def build_oracle():
 def main():
     build_hip()
     build_fortran()
+    build_pack()
     build_oracle()
 
 

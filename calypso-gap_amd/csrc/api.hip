@@ -386,6 +386,47 @@ struct DevMem {
   unsigned gen = 0;  // bumped on every (re)allocation
 };
 
+// Pinned host memory of a context, grown on demand and kept until the context
+// is freed: transfers go through it in one copy each way, without the
+// runtime's own staging of pageable memory and without waiting for the upload
+// (64 atoms: load 35 -> 12 us, results 85 -> 36 us; 67,647 atoms: 268 -> 108 and
+// 195 -> 132 us).  Starts as a part of the context's one pinned block (owned
+// false: an allocation of its own costs a new context about 50 us).
+constexpr size_t kPinnedPart = 256 * 1024;
+struct HostMem {
+  unsigned char *p = nullptr;
+  size_t cap = 0;
+  bool owned = false;
+  void release() {
+    if (p && owned) hipHostFree(p);
+    p = nullptr;
+    cap = 0;
+    owned = false;
+  }
+  int need(size_t bytes) {
+    if (bytes <= cap) return GAPX_OK;
+    release();
+    const size_t want = bytes + bytes / 8;
+    if (hipHostMalloc((void **)&p, want, hipHostMallocDefault) != hipSuccess) {
+      p = nullptr;
+      return fail(GAPX_ERR_NOMEM, "pinned host allocation failed");
+    }
+    cap = want;
+    owned = true;
+    return GAPX_OK;
+  }
+};
+
+// Byte offsets of consecutive arrays in one block, each on 256 bytes.
+struct BlockLayout {
+  size_t bytes = 0;
+  size_t add(size_t n) {
+    const size_t at = bytes;
+    bytes = (at + n + 255) / 256 * 256;
+    return at;
+  }
+};
+
 enum Stage { kNeighbors, kDescFwd, kContraction, kFinish, kDescBwd, kForces, kNumStages };
 static const char *kStageNames[kNumStages] = {"neighbor_list", "descriptors_fwd", "gpr_contraction",
                                               "gpr_finish", "descriptors_bwd", "forces_stress"};
@@ -421,6 +462,17 @@ struct Ctx {
   std::map<std::string, DevMem> mem;
   size_t bytes = 0;
   int kcap = 64, KP = 64, tcap = 1024;
+  // the loaded batch in one device block, filled by one copy from `up`
+  double *d_pos = nullptr;
+  int *d_species = nullptr, *d_astruct = nullptr;
+  StructParams *d_sp = nullptr;
+  int2 *d_map = nullptr;
+  size_t at_pos = 0, at_sp = 0;   // offsets of d_pos and d_sp in that block
+  HostMem up, down;               // staging of the batch and of the results
+  hipEvent_t up_ev = nullptr;     // the last copy out of `up`
+  // results in one device block, fetched by one copy: energies, stress,
+  // forces, per-atom energies (Np of them)
+  double *d_ene = nullptr, *d_stress = nullptr, *d_force = nullptr, *d_eatom = nullptr;
   int *host_stats = nullptr;      // pinned: the last run's list statistics
   int *host_stats_dev = nullptr;  // its device-side address
   int last_flags = -1;
@@ -700,49 +752,68 @@ static int ctx_load_batch(Ctx &c, int nstruct, const int *natoms, const int *spe
   c.Np = round_up(c.N, 128);  // row tiles of the contraction kernels
   // species must be listed in the model header (the reference leaves their
   // weight undefined, gap_calc.f90:73-83)
-  std::vector<int> listed(kMaxSpeciesZ, 0);
-  for (int k = 0; k < c.m->nspecies; ++k) listed[c.m->z[k]] = 1;
+  bool listed[kMaxSpeciesZ] = {};
+  for (int k = 0; k < c.m->nspecies; ++k) listed[c.m->z[k]] = true;
   for (int i = 0; i < c.N; ++i)
-    if (species[i] < 0 || species[i] >= kMaxSpeciesZ || !listed[species[i]]) {
+    if ((unsigned)species[i] >= (unsigned)kMaxSpeciesZ || !listed[species[i]]) {
       char buf[128];
       std::snprintf(buf, sizeof buf, "atom %d has atomic number %d, which the model does not list", i + 1, species[i]);
       return fail(GAPX_ERR_SPECIES, buf);
     }
   c.lat.resize(9 * nstruct);
-  std::vector<double> hpos(3 * (size_t)c.N);
   if (fortran) {  // single structure: LAT(3,3) and POS(NA,3) column-major
     for (int k = 0; k < 3; ++k)
       for (int x = 0; x < 3; ++x) c.lat[3 * k + x] = lat[k + 3 * x];
-    for (int i = 0; i < c.N; ++i)
-      for (int x = 0; x < 3; ++x) hpos[3 * (size_t)i + x] = pos[i + (size_t)c.N * x];
   } else {
     std::memcpy(c.lat.data(), lat, 9 * sizeof(double) * nstruct);
-    std::memcpy(hpos.data(), pos, 3 * sizeof(double) * c.N);
   }
   int rc = struct_params(c);
   if (rc) return rc;
-  std::vector<int> astruct(c.N);
-  for (int s = 0; s < nstruct; ++s)
-    for (int i = c.offsets[s]; i < c.offsets[s + 1]; ++i) astruct[i] = s;
-  int *d_species, *d_astruct;
-  double *d_pos;
-  StructParams *d_sp;
-  if ((rc = c.get("species", c.N, &d_species)) || (rc = c.get("astruct", c.N, &d_astruct)) ||
-      (rc = c.get("pos", 3 * (size_t)c.N, &d_pos)) || (rc = c.get("sp", nstruct, &d_sp)))
-    return rc;
-  GAPX_HIP(hipMemcpyAsync(d_species, species, sizeof(int) * c.N, hipMemcpyHostToDevice, c.stream));
-  GAPX_HIP(hipMemcpyAsync(d_astruct, astruct.data(), sizeof(int) * c.N, hipMemcpyHostToDevice, c.stream));
-  GAPX_HIP(hipMemcpyAsync(d_pos, hpos.data(), sizeof(double) * 3 * c.N, hipMemcpyHostToDevice, c.stream));
-  GAPX_HIP(hipMemcpyAsync(d_sp, c.sp.data(), sizeof(StructParams) * nstruct, hipMemcpyHostToDevice, c.stream));
   // the reduction's structure parts (kReduceAtoms atoms each, consecutive per structure)
-  std::vector<int2> part_map;
-  for (int s = 0; s < nstruct; ++s)
-    for (int p = 0; p * kReduceAtoms < std::max(1, c.natoms[s]); ++p) part_map.push_back(make_int2(s, p));
-  int2 *d_map;
-  if ((rc = c.get("red_map", part_map.size(), &d_map))) return rc;
-  GAPX_HIP(hipMemcpyAsync(d_map, part_map.data(), sizeof(int2) * part_map.size(), hipMemcpyHostToDevice, c.stream));
-  c.red_parts = (int)part_map.size();
-  GAPX_HIP(hipStreamSynchronize(c.stream));
+  size_t parts = 0;
+  for (int s = 0; s < nstruct; ++s) parts += (natoms[s] + kReduceAtoms - 1) / kReduceAtoms;
+  // the batch as one block: assembled in pinned memory (after the previous
+  // copy out of it), one copy to the device
+  BlockLayout in;
+  const size_t n = (size_t)c.N;
+  c.at_pos = in.add(3 * sizeof(double) * n);
+  c.at_sp = in.add(sizeof(StructParams) * nstruct);
+  const size_t at_species = in.add(sizeof(int) * n), at_astruct = in.add(sizeof(int) * n);
+  const size_t at_map = in.add(sizeof(int2) * parts);
+  GAPX_HIP(hipEventSynchronize(c.up_ev));
+  if ((rc = c.up.need(in.bytes))) return rc;
+  double *hpos = (double *)(c.up.p + c.at_pos);
+  if (fortran) {
+    for (int i = 0; i < c.N; ++i)
+      for (int x = 0; x < 3; ++x) hpos[3 * (size_t)i + x] = pos[i + (size_t)c.N * x];
+  } else {
+    std::memcpy(hpos, pos, 3 * sizeof(double) * n);
+  }
+  std::memcpy(c.up.p + c.at_sp, c.sp.data(), sizeof(StructParams) * nstruct);
+  std::memcpy(c.up.p + at_species, species, sizeof(int) * n);
+  int *astruct = (int *)(c.up.p + at_astruct);
+  int2 *map = (int2 *)(c.up.p + at_map);
+  for (int s = 0; s < nstruct; ++s) {
+    std::fill(astruct + c.offsets[s], astruct + c.offsets[s + 1], s);
+    for (int p = 0; p * kReduceAtoms < natoms[s]; ++p) *map++ = make_int2(s, p);
+  }
+  c.red_parts = (int)parts;
+  unsigned char *d_in, *d_out;
+  BlockLayout out;
+  const size_t at_ene = out.add(sizeof(double) * nstruct), at_stress = out.add(6 * sizeof(double) * nstruct);
+  const size_t at_force = out.add(3 * sizeof(double) * n), at_eatom = out.add(sizeof(double) * c.Np);
+  if ((rc = c.get("in", in.bytes, &d_in)) || (rc = c.get("out", out.bytes, &d_out))) return rc;
+  GAPX_HIP(hipMemcpyAsync(d_in, c.up.p, in.bytes, hipMemcpyHostToDevice, c.stream));
+  GAPX_HIP(hipEventRecord(c.up_ev, c.stream));
+  c.d_pos = (double *)(d_in + c.at_pos);
+  c.d_sp = (StructParams *)(d_in + c.at_sp);
+  c.d_species = (int *)(d_in + at_species);
+  c.d_astruct = (int *)(d_in + at_astruct);
+  c.d_map = (int2 *)(d_in + at_map);
+  c.d_ene = (double *)(d_out + at_ene);
+  c.d_stress = (double *)(d_out + at_stress);
+  c.d_force = (double *)(d_out + at_force);
+  c.d_eatom = (double *)(d_out + at_eatom);
   c.kcap = initial_kcap(c);
   c.tcap = initial_tcap(c);
   default_tuning(c);
@@ -839,9 +910,9 @@ static int run_neighbors(Ctx &c, int flags, Bufs &b) {
     if ((rc = c.get("fc_scratch", tbytes, &t))) return rc;
     nb.fc_scratch = t;
   }
-  const int *d_astruct = c.ptr<int>("astruct");
-  const double *d_pos = c.ptr<double>("pos");
-  const StructParams *d_sp = c.ptr<StructParams>("sp");
+  const int *d_astruct = c.d_astruct;
+  const double *d_pos = c.d_pos;
+  const StructParams *d_sp = c.d_sp;
   if (c.fused_bins) {
     GAPX_HIP(launch_bin_structures(c.stream, c.nstruct, d_pos, d_sp, nb, c.nbins, c.fused_atoms, c.fused_bins_max,
                                    stats));
@@ -883,8 +954,15 @@ static int run_neighbors(Ctx &c, int flags, Bufs &b) {
 // With per-stage timing on, every stage runs alone on the work stream and
 // the map is built inside the neighbour stage instead (reverse_in_timing), so
 // that each stage's time is its own kernels' time.
+// Small batches build it in line: the map takes about 6 us there, less than the
+// two cross-stream dependencies.
+static bool reverse_in_line(const Ctx &c) { return c.N <= 2048; }
 static int fork_reverse(Ctx &c, Bufs &b) {
   if (c.timing) return GAPX_OK;
+  if (reverse_in_line(c)) {
+    GAPX_HIP(launch_reverse_slots(c.stream, c.N, b.nb));
+    return GAPX_OK;
+  }
   GAPX_HIP(hipEventRecord(c.fork_ev, c.stream));
   GAPX_HIP(hipStreamWaitEvent(c.aux, c.fork_ev, 0));
   GAPX_HIP(launch_reverse_slots(c.aux, c.N, b.nb));
@@ -924,9 +1002,10 @@ static int gpr_layout(Ctx &c, GprArgs &g, bool f64_kernel, int tune) {
 // per-structure energy and virial, list statistics.
 static int forces_buffers(Ctx &c, Bufs &b, bool grad) {
   int rc;
-  if ((rc = c.get("force", 3 * (size_t)c.N, &b.force)) || (rc = c.get("ene", c.nstruct, &b.ene)) ||
-      (rc = c.get("stress", 6 * (size_t)c.nstruct, &b.stress)) || (rc = c.get("atom_vir", 6 * (size_t)c.N, &b.atom_vir)))
-    return rc;
+  b.force = c.d_force;
+  b.ene = c.d_ene;
+  b.stress = c.d_stress;
+  if ((rc = c.get("atom_vir", 6 * (size_t)c.N, &b.atom_vir))) return rc;
   if (grad && (rc = c.get("slot_f", 3 * (size_t)c.N * c.kcap, &b.slot_f))) return rc;
   return GAPX_OK;
 }
@@ -935,7 +1014,7 @@ static int forces_buffers(Ctx &c, Bufs &b, bool grad) {
 static int enqueue_bwd(Ctx &c, Bufs &b, bool fp64, const GradSrc &gs, int waves_bwd, hipStream_t s, int atom0,
                        int count) {
   Model &m = *c.m;
-  GAPX_HIP(launch_descriptors_bwd(s, fp64, count, c.ptr<int>("species"), m.d_wz, b.nb, b.tb, m.sfd, m.Dp, gs,
+  GAPX_HIP(launch_descriptors_bwd(s, fp64, count, c.d_species, m.d_wz, b.nb, b.tb, m.sfd, m.Dp, gs,
                                   b.slot_f, b.atom_vir, waves_bwd, c.KP, atom0));
   return GAPX_OK;
 }
@@ -943,7 +1022,7 @@ static int enqueue_bwd(Ctx &c, Bufs &b, bool fp64, const GradSrc &gs, int waves_
 static int enqueue_forces(Ctx &c, Bufs &b, bool fp64, bool grad, const double *eatom, const GradSrc &gs,
                           int waves_bwd, bool bwd_done = false) {
   NeighborBufs &nb = b.nb;
-  const StructParams *d_sp = c.ptr<StructParams>("sp");
+  const StructParams *d_sp = c.d_sp;
   int rc;
   if ((rc = forces_buffers(c, b, grad))) return rc;
   if (grad && !bwd_done) {
@@ -970,14 +1049,14 @@ static int enqueue_forces(Ctx &c, Bufs &b, bool fp64, bool grad, const double *e
       c.red_clean = g;
     }
   }
-  rb.part_map = c.ptr<int2>("red_map");
+  rb.part_map = c.d_map;
   rb.nparts = c.red_parts;
   rb.part_sum = part_sum;
   rb.ticket = ticket;
   rb.stats_acc = stats_acc;
   rb.sticky = stats_acc + 8;
   rb.overflow_now = stats_acc + 16;
-  if (grad && !c.timing) GAPX_HIP(hipStreamWaitEvent(c.stream, c.join_ev, 0));
+  if (grad && !c.timing && !reverse_in_line(c)) GAPX_HIP(hipStreamWaitEvent(c.stream, c.join_ev, 0));
   stage_begin(c, kForces);
   GAPX_HIP(launch_forces_reduce(c.stream, c.N, grad ? 1 : 0, nb, b.slot_f, !fp64, b.force, c.nstruct, d_sp, eatom,
                                 b.atom_vir, b.ene, b.stress, b.tb, rb, c.host_stats_dev));
@@ -998,7 +1077,7 @@ static int enqueue_run(Ctx &c, int flags) {
   stage_begin(c, kNeighbors);
   if ((rc = run_neighbors(c, flags, b)) || (rc = reverse_in_timing(c, b, grad))) return rc;
   NeighborBufs &nb = b.nb;
-  const int *d_species = c.ptr<int>("species");
+  const int *d_species = c.d_species;
   stage_end(c, kNeighbors);
 
   // descriptors
@@ -1060,7 +1139,8 @@ static int enqueue_run(Ctx &c, int flags) {
   g.grad = grad ? 1 : 0;
   g.bf16 = bf ? 1 : 0;
   g.wscale = m.w_scale;
-  if ((rc = c.get("Epart", (size_t)g.splits * c.Np, &g.Epart)) || (rc = c.get("eatom", c.Np, &g.eatom))) return rc;
+  if ((rc = c.get("Epart", (size_t)g.splits * c.Np, &g.Epart))) return rc;
+  g.eatom = c.d_eatom;
   if (grad) {
     if (c64) {
       if ((rc = c.get("Gpart", (size_t)g.splits * ND, &g.Gpart))) return rc;
@@ -1176,7 +1256,7 @@ static int enqueue_surrogate(Ctx &c, Mlp &mlp, int flags) {
   }
   const Tuning &tu = c.tune[fp64 ? 0 : 1];
   stage_begin(c, kDescFwd);
-  GAPX_HIP(launch_descriptors_fwd(c.stream, fp64, c.N, c.ptr<int>("species"), m.d_wz, b.nb, b.tb, m.sfd,
+  GAPX_HIP(launch_descriptors_fwd(c.stream, fp64, c.N, c.d_species, m.d_wz, b.nb, b.tb, m.sfd,
                                   m.d_theta_inv, m.d_mu, 0, o, c.chunk > 0 ? c.chunk : 16, tu.waves_fwd, c.KP));
   stage_end(c, kDescFwd);
   if (grad && (rc = fork_reverse(c, b))) return rc;
@@ -1186,9 +1266,8 @@ static int enqueue_surrogate(Ctx &c, Mlp &mlp, int flags) {
     GAPX_HIP(launch_f64_to_f32(c.stream, (size_t)c.N * Dp, o.xt64, xin));
   }
   if (c.Np > c.N) GAPX_HIP(launch_fill_int(c.stream, (int *)(xin + (size_t)c.N * Dp), (c.Np - c.N) * Dp, 0));
-  double *eatom = nullptr, *g64 = nullptr;
+  double *eatom = c.d_eatom, *g64 = nullptr;
   float *g32 = nullptr;
-  if ((rc = c.get("eatom", c.Np, &eatom))) return rc;
   if (grad) {
     if (fp64) {
       if ((rc = c.get("g64", ND, &g64))) return rc;
@@ -1293,13 +1372,16 @@ static int capacity_verdict(Ctx &c, const int *h, int kroom, int troom, bool *gr
   return GAPX_OK;
 }
 
-static int ctx_settle(Ctx &c) {
+// *repeated (may be null): whether the run was enqueued again.
+static int ctx_settle(Ctx &c, bool *repeated = nullptr) {
+  if (repeated) *repeated = false;
   GAPX_HIP(hipStreamSynchronize(c.stream));
   collect_timing(c);
   for (int attempt = 0; attempt < 4; ++attempt) {
     bool grow;
     int rc = capacity_verdict(c, c.host_stats, 8, 64, &grow);
     if (rc || !grow) return rc;
+    if (repeated) *repeated = true;
     if ((rc = ctx_run(c, c.last_flags, c.mlp))) return rc;
     GAPX_HIP(hipStreamSynchronize(c.stream));
     collect_timing(c);
@@ -1570,8 +1652,8 @@ static int ctx_relax(Ctx &c, int flags, int max_steps, double fmax, double maxst
   if ((rc = ctx_run(c, flags)) || (rc = ctx_settle(c))) return rc;  // forces at the start
   trajectory_headroom(c);
   auto step = [&](StepCtl ctl) {
-    return launch_fire_step(c.stream, c.nstruct, c.N, c.ptr<StructParams>("sp"), c.ptr<int>("astruct"),
-                            c.ptr<double>("force"), vel, c.ptr<double>("pos"), st, fp, ctl);
+    return launch_fire_step(c.stream, c.nstruct, c.N, c.d_sp, c.d_astruct,
+                            c.d_force, vel, c.d_pos, st, fp, ctl);
   };
   auto fetch = [&](int *conv) {
     GAPX_HIP(hipMemcpyAsync(hs.data(), st, sizeof(FireState) * c.nstruct, hipMemcpyDeviceToHost, c.stream));
@@ -1607,8 +1689,8 @@ static int ctx_relax_lbfgs(Ctx &c, int flags, int max_steps, double fmax, double
   if ((rc = ctx_run(c, flags)) || (rc = ctx_settle(c))) return rc;  // forces at the start
   trajectory_headroom(c);
   auto launch = [&](StepCtl ctl, const LbfgsParams &p) {
-    return launch_lbfgs_step(c.stream, c.nstruct, c.N, c.ptr<StructParams>("sp"), c.ptr<double>("force"),
-                             c.ptr<double>("pos"), r0, f0, S, Y, rho, q, st, p, ctl);
+    return launch_lbfgs_step(c.stream, c.nstruct, c.N, c.d_sp, c.d_force,
+                             c.d_pos, r0, f0, S, Y, rho, q, st, p, ctl);
   };
   auto fetch = [&](int *conv) {
     GAPX_HIP(hipMemcpyAsync(hs.data(), st, sizeof(LbfgsState) * c.nstruct, hipMemcpyDeviceToHost, c.stream));
@@ -1672,32 +1754,32 @@ static int ctx_md(Ctx &c, int flags, int nsteps, double dt, double temperature, 
   else
     GAPX_HIP(launch_fill_double(c.stream, p, n3, 0.0));
   const MdParams mp{dt, temperature, taut, kBoltzmannEv, fixcm ? 1 : 0, 0};
-  const StructParams *d_sp = c.ptr<StructParams>("sp");
-  const int *d_as = c.ptr<int>("astruct");
+  const StructParams *d_sp = c.d_sp;
+  const int *d_as = c.d_astruct;
   if ((rc = ctx_run(c, flags)) || (rc = ctx_settle(c))) return rc;
   trajectory_headroom(c);
-  if (dlog) GAPX_HIP(launch_md_log(c.stream, c.nstruct, d_sp, mass, p, c.ptr<double>("force"), c.ptr<double>("ene"),
+  if (dlog) GAPX_HIP(launch_md_log(c.stream, c.nstruct, d_sp, mass, p, c.d_force, c.d_ene,
                                    mp.kB, dlog));
   int hs[8];
   for (int b0 = 0, redo = 0; b0 < nsteps;) {
     const int nb = std::min(kMdCheckEvery, nsteps - b0);
     // the block's starting state, and a cleared running maximum
-    GAPX_HIP(hipMemcpyAsync(ck_x, c.ptr<double>("pos"), sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
+    GAPX_HIP(hipMemcpyAsync(ck_x, c.d_pos, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
     GAPX_HIP(hipMemcpyAsync(ck_p, p, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
-    GAPX_HIP(hipMemcpyAsync(ck_f, c.ptr<double>("force"), sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
-    GAPX_HIP(hipMemcpyAsync(ck_e, c.ptr<double>("ene"), sizeof(double) * c.nstruct, hipMemcpyDeviceToDevice,
+    GAPX_HIP(hipMemcpyAsync(ck_f, c.d_force, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
+    GAPX_HIP(hipMemcpyAsync(ck_e, c.d_ene, sizeof(double) * c.nstruct, hipMemcpyDeviceToDevice,
                             c.stream));
     int *sticky = c.ptr<int>("stats_acc") + 8;
     GAPX_HIP(launch_fill_int(c.stream, sticky, 8, 0));
     for (int step = b0; step < b0 + nb; ++step) {
-      double *x = c.ptr<double>("pos"), *f = c.ptr<double>("force");
+      double *x = c.d_pos, *f = c.d_force;
       GAPX_HIP(launch_md_prepare(c.stream, c.nstruct, d_sp, mass, p, f, mp, coef));
       GAPX_HIP(launch_md_drift(c.stream, c.N, d_as, mass, f, coef, dt, p, x));
       if ((rc = ctx_run(c, flags))) return rc;
-      f = c.ptr<double>("force");
+      f = c.d_force;
       GAPX_HIP(launch_md_kick(c.stream, c.N, f, 0.5 * dt, p));
       if (dlog)
-        GAPX_HIP(launch_md_log(c.stream, c.nstruct, d_sp, mass, p, f, c.ptr<double>("ene"), mp.kB,
+        GAPX_HIP(launch_md_log(c.stream, c.nstruct, d_sp, mass, p, f, c.d_ene, mp.kB,
                                dlog + 3 * (size_t)c.nstruct * (step + 1)));
     }
     sticky = c.ptr<int>("stats_acc") + 8;
@@ -1714,10 +1796,10 @@ static int ctx_md(Ctx &c, int flags, int nsteps, double dt, double temperature, 
     if (++redo > 3) return fail(GAPX_ERR_NEIGHBORS, "neighbour capacity did not converge during MD");
     // back to the block's start (buffers of the run's size class are not
     // reallocated by a capacity change, so the saved state still applies)
-    GAPX_HIP(hipMemcpyAsync(c.ptr<double>("pos"), ck_x, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
+    GAPX_HIP(hipMemcpyAsync(c.d_pos, ck_x, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
     GAPX_HIP(hipMemcpyAsync(p, ck_p, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
-    GAPX_HIP(hipMemcpyAsync(c.ptr<double>("force"), ck_f, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
-    GAPX_HIP(hipMemcpyAsync(c.ptr<double>("ene"), ck_e, sizeof(double) * c.nstruct, hipMemcpyDeviceToDevice,
+    GAPX_HIP(hipMemcpyAsync(c.d_force, ck_f, sizeof(double) * n3, hipMemcpyDeviceToDevice, c.stream));
+    GAPX_HIP(hipMemcpyAsync(c.d_ene, ck_e, sizeof(double) * c.nstruct, hipMemcpyDeviceToDevice,
                             c.stream));
   }
   if (log)
@@ -1730,17 +1812,28 @@ static int ctx_md(Ctx &c, int flags, int nsteps, double dt, double temperature, 
 
 static int ctx_results(Ctx &c, double *ene, double *force, double *stress6, double *eatom, bool fortran) {
   if (!c.ran) return fail(GAPX_ERR_ARG, "no evaluation has run on this context");
-  int rc = ctx_settle(c);
+  // the leading part of the results' block that holds what is asked for, in
+  // one copy behind the run; a run repeated with larger lists copies again
+  auto at = [&](const double *p) { return (size_t)((const unsigned char *)p - (const unsigned char *)c.d_ene); };
+  const size_t bytes = eatom   ? at(c.d_eatom) + sizeof(double) * c.N
+                       : force ? at(c.d_force) + 3 * sizeof(double) * c.N
+                               : at(c.d_stress) + 6 * sizeof(double) * c.nstruct;
+  int rc = c.down.need(bytes);
   if (rc) return rc;
-  if (ene) GAPX_HIP(hipMemcpy(ene, c.ptr<double>("ene"), sizeof(double) * c.nstruct, hipMemcpyDeviceToHost));
-  if (stress6) GAPX_HIP(hipMemcpy(stress6, c.ptr<double>("stress"), sizeof(double) * 6 * c.nstruct, hipMemcpyDeviceToHost));
-  if (eatom) GAPX_HIP(hipMemcpy(eatom, c.ptr<double>("eatom"), sizeof(double) * c.N, hipMemcpyDeviceToHost));
+  bool repeated = true;
+  while (repeated) {
+    GAPX_HIP(hipMemcpyAsync(c.down.p, c.d_ene, bytes, hipMemcpyDeviceToHost, c.stream));
+    if ((rc = ctx_settle(c, &repeated))) return rc;
+  }
+  auto host = [&](const double *p) { return (const double *)(c.down.p + at(p)); };
+  if (ene) std::memcpy(ene, host(c.d_ene), sizeof(double) * c.nstruct);
+  if (stress6) std::memcpy(stress6, host(c.d_stress), 6 * sizeof(double) * c.nstruct);
+  if (eatom) std::memcpy(eatom, host(c.d_eatom), sizeof(double) * c.N);
   if (force) {
+    const double *f = host(c.d_force);
     if (!fortran) {
-      GAPX_HIP(hipMemcpy(force, c.ptr<double>("force"), sizeof(double) * 3 * c.N, hipMemcpyDeviceToHost));
+      std::memcpy(force, f, 3 * sizeof(double) * c.N);
     } else {
-      std::vector<double> f(3 * (size_t)c.N);
-      GAPX_HIP(hipMemcpy(f.data(), c.ptr<double>("force"), sizeof(double) * 3 * c.N, hipMemcpyDeviceToHost));
       for (int i = 0; i < c.N; ++i)
         for (int x = 0; x < 3; ++x) force[i + (size_t)c.N * x] = f[3 * (size_t)i + x];
     }
@@ -1768,7 +1861,7 @@ static int ctx_variance(Ctx &c, double *var, double *sigma2) {
   v.mt = m.d_mt;
   v.mn = m.d_mn;
   v.qmm = m.d_qmm;
-  v.sp = c.ptr<StructParams>("sp");
+  v.sp = c.d_sp;
   if ((rc = c.get("var_sigma2", c.N, &v.sigma2)) || (rc = c.get("var_struct", c.nstruct, &v.var))) return rc;
   if (v.qmm) {
     if ((rc = c.get("var_xn", c.N, &v.xn)) || (rc = c.get("var_K", (size_t)v.rows * m.Mp, &v.K)) ||
@@ -1939,19 +2032,24 @@ static int ctx_create(Model *m, Ctx **out) {
   if (hipStreamCreateWithFlags(&c->aux, hipStreamNonBlocking) != hipSuccess ||
       hipStreamCreateWithFlags(&c->aux2, hipStreamNonBlocking) != hipSuccess ||
       hipEventCreateWithFlags(&c->fork_ev, hipEventDisableTiming) != hipSuccess ||
+      hipEventCreateWithFlags(&c->up_ev, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&c->join_ev, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&c->half_ev, hipEventDisableTiming) != hipSuccess ||
       hipEventCreateWithFlags(&c->half_done_ev, hipEventDisableTiming) != hipSuccess) {
     ctx_free(c);
     return fail(GAPX_ERR_HIP, "could not create the second stream or its events");
   }
-  if (hipHostMalloc((void **)&c->host_stats, 8 * sizeof(int), hipHostMallocMapped | hipHostMallocCoherent) !=
+  // the statistics, then the first room of both transfer stagings
+  if (hipHostMalloc((void **)&c->host_stats, 256 + 2 * kPinnedPart, hipHostMallocMapped | hipHostMallocCoherent) !=
           hipSuccess ||
       hipHostGetDevicePointer((void **)&c->host_stats_dev, c->host_stats, 0) != hipSuccess) {
     ctx_free(c);
     return fail(GAPX_ERR_NOMEM, "pinned host allocation failed");
   }
   std::memset(c->host_stats, 0, 8 * sizeof(int));
+  c->up.p = (unsigned char *)c->host_stats + 256;
+  c->down.p = c->up.p + kPinnedPart;
+  c->up.cap = c->down.cap = kPinnedPart;
   // Shapes before the first load (default_tuning sets them by the batch):
   // one wavefront per atom for grid-form tables, four for generic ones;
   // 128-row tiles for the mixed contraction.
@@ -1985,6 +2083,9 @@ static void ctx_free(Ctx *c) {
   if (c->join_ev) hipEventDestroy(c->join_ev);
   if (c->half_ev) hipEventDestroy(c->half_ev);
   if (c->half_done_ev) hipEventDestroy(c->half_done_ev);
+  if (c->up_ev) hipEventDestroy(c->up_ev);
+  c->up.release();
+  c->down.release();
   if (c->host_stats) hipHostFree(c->host_stats);
   delete c;
 }
@@ -2567,11 +2668,18 @@ int gapx_ctx_update(gapx_ctx *c, const double *lat, const double *pos) {
     }
     // a captured graph whose binning launch parameters no longer match is
     // replaced at the next run (Ctx::graph_matches)
-    GAPX_HIP(hipMemcpyAsync(c->ptr<StructParams>("sp"), c->sp.data(), sizeof(StructParams) * c->nstruct,
-                            hipMemcpyHostToDevice, c->stream));
   }
-  GAPX_HIP(hipMemcpyAsync(c->ptr<double>("pos"), pos, sizeof(double) * 3 * c->N, hipMemcpyHostToDevice, c->stream));
-  GAPX_HIP(hipStreamSynchronize(c->stream));
+  // through the pinned block, once the previous copy out of it is done; the
+  // device copy is ordered on the stream, so nothing waits for it here
+  GAPX_HIP(hipEventSynchronize(c->up_ev));
+  std::memcpy(c->up.p + c->at_pos, pos, sizeof(double) * 3 * c->N);
+  GAPX_HIP(hipMemcpyAsync(c->d_pos, c->up.p + c->at_pos, sizeof(double) * 3 * c->N, hipMemcpyHostToDevice, c->stream));
+  if (lat) {
+    std::memcpy(c->up.p + c->at_sp, c->sp.data(), sizeof(StructParams) * c->nstruct);
+    GAPX_HIP(hipMemcpyAsync(c->d_sp, c->up.p + c->at_sp, sizeof(StructParams) * c->nstruct, hipMemcpyHostToDevice,
+                            c->stream));
+  }
+  GAPX_HIP(hipEventRecord(c->up_ev, c->stream));
   return GAPX_OK;
 }
 
@@ -2694,7 +2802,7 @@ int gapx_ctx_export_labels(gapx_ctx *c, gapx_mlp *m) {
   const bool fp64 = !(c->last_flags & GAPX_MIXED);
   return mlp_add_labels(*mlp_of(m), c->stream, c->N, fp64 ? nullptr : c->ptr<float>("xt32"),
                         fp64 ? c->ptr<double>("xt64") : nullptr, fp64 ? nullptr : c->ptr<float>("g32"),
-                        fp64 ? c->ptr<double>("g64") : nullptr, c->ptr<double>("eatom"), c->m->d_theta_inv, c->m->Dp);
+                        fp64 ? c->ptr<double>("g64") : nullptr, c->d_eatom, c->m->d_theta_inv, c->m->Dp);
 }
 
 int gapx_ctx_relax(gapx_ctx *c, int flags, int max_steps, double fmax, double maxstep, int *steps_done,
@@ -2715,7 +2823,7 @@ int gapx_ctx_positions(gapx_ctx *c, double *pos) {
   if (!c || !pos || c->N <= 0) return fail(GAPX_ERR_ARG, "gapx_ctx_positions: nothing loaded");
   GAPX_HIP(hipSetDevice(c->device));
   GAPX_HIP(hipStreamSynchronize(c->stream));
-  GAPX_HIP(hipMemcpy(pos, c->ptr<double>("pos"), sizeof(double) * 3 * c->N, hipMemcpyDeviceToHost));
+  GAPX_HIP(hipMemcpy(pos, c->d_pos, sizeof(double) * 3 * c->N, hipMemcpyDeviceToHost));
   return GAPX_OK;
 }
 

@@ -143,6 +143,42 @@ def _p(a):
     return ctypes.c_void_p(a.ctypes.data) if a is not None else ctypes.c_void_p(0)
 
 
+try:
+    from . import _pack
+except ImportError:  # not built: the numpy concatenations below
+    _pack = None
+
+
+class _Batch:
+    """Structures packed back to back for the C ABI, in arrays kept between loads."""
+
+    def __init__(self):
+        self.natoms = np.empty(0, np.int32)
+        self.species = np.empty(0, np.int32)
+        self.lat = np.empty(0)
+        self.pos = np.empty(0)
+
+    def pack(self, structures):
+        """(natoms, species, lat, pos) of a list of dicts with "species", "lat" and "pos"."""
+        n = len(structures)
+        if _pack is not None and n > 1 and isinstance(structures, list):
+            if len(self.natoms) < n:
+                self.natoms, self.lat = np.empty(n, np.int32), np.empty(9 * n)
+            total = _pack.gather(structures, self.natoms, self.species, self.lat, self.pos)
+            if total is not None and total > len(self.species):
+                self.species, self.pos = np.empty(total + total // 8, np.int32), np.empty(3 * (total + total // 8))
+                total = _pack.gather(structures, self.natoms, self.species, self.lat, self.pos)
+            if total is not None:
+                # natoms goes to the caller, who may keep it; the others are only read by the load
+                return self.natoms[:n].copy(), self.species, self.lat, self.pos
+        # other array types or layouts
+        natoms = np.array([len(s["species"]) for s in structures], np.int32)
+        species = np.ascontiguousarray(np.concatenate([s["species"] for s in structures]), np.int32)
+        lat = np.ascontiguousarray(np.stack([s["lat"] for s in structures]), np.float64)
+        pos = np.ascontiguousarray(np.concatenate([s["pos"] for s in structures]), np.float64)
+        return natoms, species, lat, pos
+
+
 def device_count():
     n = ctypes.c_int(0)
     _check(lib().gapx_device_count(ctypes.byref(n)))
@@ -170,6 +206,7 @@ class Model:
 
     def __init__(self, handle):
         self._h = ctypes.c_void_p(handle)
+        self._batch = _Batch()
         ns, nsf, D, M = (ctypes.c_int() for _ in range(4))
         _check(lib().gapx_model_dims(self._h, ctypes.byref(ns), ctypes.byref(nsf), ctypes.byref(D),
                                      ctypes.byref(M)))
@@ -257,10 +294,7 @@ class Model:
         return float(ene[0]), force, stress, float(var[0])
 
     def calc_batch(self, structures, rcut=6.0, grad=True, mixed=False, flags=0):
-        natoms = np.array([len(s["species"]) for s in structures], np.int32)
-        species = np.ascontiguousarray(np.concatenate([s["species"] for s in structures]), np.int32)
-        lat = np.ascontiguousarray(np.stack([s["lat"] for s in structures]), np.float64)
-        pos = np.ascontiguousarray(np.concatenate([s["pos"] for s in structures]), np.float64)
+        natoms, species, lat, pos = self._batch.pack(structures)
         ene = np.zeros(len(structures))
         force = np.zeros((int(natoms.sum()), 3))
         stress = np.zeros((len(structures), 6))
@@ -334,14 +368,12 @@ class Context:
         h = ctypes.c_void_p()
         _check(lib().gapx_ctx_create(model._h, ctypes.byref(h)))
         self._h = h
+        self._batch = _Batch()
         self.nstruct = 0
         self.natoms = None
 
     def load(self, structures, rcut=6.0):
-        self.natoms = np.array([len(s["species"]) for s in structures], np.int32)
-        species = np.ascontiguousarray(np.concatenate([s["species"] for s in structures]), np.int32)
-        lat = np.ascontiguousarray(np.stack([s["lat"] for s in structures]), np.float64)
-        pos = np.ascontiguousarray(np.concatenate([s["pos"] for s in structures]), np.float64)
+        self.natoms, species, lat, pos = self._batch.pack(structures)
         self.nstruct = len(structures)
         _check(lib().gapx_ctx_load(self._h, self.nstruct, _p(self.natoms), _p(species), _p(lat), _p(pos),
                                    float(rcut)))
@@ -359,10 +391,10 @@ class Context:
 
     def results(self):
         n = int(self.natoms.sum())
-        ene = np.zeros(self.nstruct)
-        force = np.zeros((n, 3))
-        stress = np.zeros((self.nstruct, 6))
-        eatom = np.zeros(n)
+        ene = np.empty(self.nstruct)
+        force = np.empty((n, 3))
+        stress = np.empty((self.nstruct, 6))
+        eatom = np.empty(n)
         _check(lib().gapx_ctx_results(self._h, _p(ene), _p(force), _p(stress), _p(eatom)))
         return dict(energy=ene, forces=force, stress=stress, eatom=eatom)
 
