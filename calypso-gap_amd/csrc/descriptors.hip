@@ -270,6 +270,47 @@ __device__ __forceinline__ void line_power(const SFDev &sf, int s, T cth, PowSta
 // row enters d2, i.e. 0 in FP32 and in FP64 alike.
 __device__ __forceinline__ double fp16_operand(double xt) { return fmin(fmax(xt, -32768.0), 32768.0); }
 
+__device__ __forceinline__ void split16(int mode, double xt, uint16_t &h, uint16_t &l) {
+  if (mode == 1) {  // FP16 hi + lo of xt clamped to the FP16 range (see fp16_operand)
+    const double xc = fp16_operand(xt);
+    const _Float16 hi = (_Float16)xc, lo = (_Float16)(xc - (double)hi);
+    h = __builtin_bit_cast(uint16_t, hi);
+    l = __builtin_bit_cast(uint16_t, lo);
+  } else {  // BF16 hi + lo
+    const __bf16 hi = (__bf16)(float)xt, lo = (__bf16)(float)(xt - (double)(float)hi);
+    h = __builtin_bit_cast(uint16_t, hi);
+    l = __builtin_bit_cast(uint16_t, lo);
+  }
+}
+
+// A row's outputs from its features in LDS, two features per thread (Dp is a
+// multiple of 32, the rows are aligned): raw features, centred and scaled ones,
+// the split operands; returns this thread's part of |xt|^2 in FP64.
+template <typename T, int W>
+__device__ __forceinline__ double write_features(const T *s_feat, size_t row, int Dp, int tid, const double *theta_inv,
+                                                 const double *mu, int split_mode, const DescOut &out) {
+  double xn = 0.0;
+  for (int d = 2 * tid; d < Dp; d += 128 * W) {
+    const T x0 = s_feat[d], x1 = s_feat[d + 1];
+    const double2 ti = *(const double2 *)(theta_inv + d), m = *(const double2 *)(mu + d);
+    const double t0 = (double)x0 * ti.x - m.x, t1 = (double)x1 * ti.y - m.y;
+    xn += t0 * t0;
+    xn += t1 * t1;
+    if (out.x64) *(double2 *)(out.x64 + row + d) = make_double2((double)x0, (double)x1);
+    if (out.x32) *(float2 *)(out.x32 + row + d) = make_float2((float)x0, (float)x1);
+    if (out.xt64) *(double2 *)(out.xt64 + row + d) = make_double2(t0, t1);
+    if (out.xt32) *(float2 *)(out.xt32 + row + d) = make_float2((float)t0, (float)t1);
+    if (split_mode) {
+      ushort2 h, l;
+      split16(split_mode, t0, h.x, l.x);
+      split16(split_mode, t1, h.y, l.y);
+      *(ushort2 *)(out.xt_hi + row + d) = h;
+      *(ushort2 *)(out.xt_lo + row + d) = l;
+    }
+  }
+  return xn;
+}
+
 // Weight of a neighbour slot: the caller's (CAR2ACSF's neighbour table), or
 // that of the neighbour's species.
 __device__ __forceinline__ double slot_weight(const NeighborBufs &nb, const double *wz, const int *species,
@@ -489,30 +530,7 @@ __global__ __launch_bounds__(W > 4 ? 64 * W : 256) void k_desc_fwd(int N, const 
     chunk_reduce<T, NCH, W>(acc, accw, wv, lane, tid, c0, sf.n_ang, sf.ang_feat, sf.nsf, s_part, s_feat);
   }
 
-  // epilogue: raw features, centred/scaled features, FP64 norm, split operands
-  double xn = 0.0;
-  const size_t row = (size_t)i * Dp;
-  for (int d = tid; d < Dp; d += 64 * W) {
-    const T x = s_feat[d];
-    if (out.x64) out.x64[row + d] = (double)x;
-    if (out.x32) out.x32[row + d] = (float)x;
-    const double xt = (double)x * theta_inv[d] - mu[d];
-    xn += xt * xt;
-    if (out.xt64) out.xt64[row + d] = xt;
-    if (out.xt32) out.xt32[row + d] = (float)xt;
-    if (split_mode == 1) {  // FP16 hi + lo of xt clamped to the FP16 range (see fp16_operand)
-      const double xc = fp16_operand(xt);
-      const _Float16 hi = (_Float16)xc;
-      const _Float16 lo = (_Float16)(xc - (double)hi);
-      out.xt_hi[row + d] = __builtin_bit_cast(uint16_t, hi);
-      out.xt_lo[row + d] = __builtin_bit_cast(uint16_t, lo);
-    } else if (split_mode == 2) {  // BF16 hi + lo
-      const __bf16 hi = (__bf16)(float)xt;
-      const __bf16 lo = (__bf16)(float)(xt - (double)(float)hi);
-      out.xt_hi[row + d] = __builtin_bit_cast(uint16_t, hi);
-      out.xt_lo[row + d] = __builtin_bit_cast(uint16_t, lo);
-    }
-  }
+  double xn = write_features<T, W>(s_feat, (size_t)i * Dp, Dp, tid, theta_inv, mu, split_mode, out);
   xn = wave_sum(xn);
   if (lane == 0) s_xn[wv] = xn;
   __syncthreads();
@@ -650,6 +668,33 @@ __device__ __forceinline__ double swap_sum(double a, double b) {
          __longlong_as_double((long long)(((unsigned long long)vh << 32) | vl));
 }
 
+// The value of the lane at l ^ M for M = 8, 4, 2, 1 (within a row of 16 lanes)
+// by cross-lane moves of the vector units instead of a trip through LDS: a row
+// rotation by 8, quad permutations for 1 and 2, and for 4 the reversal of each
+// half row (l ^ 7) after that of each quad (l ^ 3).
+template <int CTRL>
+__device__ __forceinline__ unsigned dpp32(unsigned v) {
+  return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true);
+}
+template <int M>
+__device__ __forceinline__ unsigned lane_xor(unsigned v) {
+  static_assert(M == 8 || M == 4 || M == 2 || M == 1, "within a row");
+  if constexpr (M == 8) return dpp32<0x128>(v);                // row_ror:8
+  if constexpr (M == 4) return dpp32<0x141>(dpp32<0x1B>(v));   // quad_perm:[3,2,1,0], row_half_mirror
+  if constexpr (M == 2) return dpp32<0x4E>(v);                 // quad_perm:[2,3,0,1]
+  return dpp32<0xB1>(v);                                       // quad_perm:[1,0,3,2]
+}
+template <int M>
+__device__ __forceinline__ float lane_xor(float v) {
+  return __uint_as_float(lane_xor<M>(__float_as_uint(v)));
+}
+template <int M>
+__device__ __forceinline__ double lane_xor(double v) {
+  const unsigned long long u = __double_as_longlong(v);
+  const unsigned lo = lane_xor<M>((unsigned)u), hi = lane_xor<M>((unsigned)(u >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 template <typename T, int M, int NVP>
 __device__ __forceinline__ void butterfly(T (&x)[NVP], int lane) {
   if constexpr (M == 32 || M == 16) {
@@ -662,7 +707,7 @@ __device__ __forceinline__ void butterfly(T (&x)[NVP], int lane) {
     for (int j = 0; j < M; ++j) {
       const T send = upper ? x[j] : x[j + M];
       const T keep = upper ? x[j + M] : x[j];
-      x[j] = keep + __shfl_xor(send, M, 64);
+      x[j] = keep + lane_xor<M>(send);
     }
     butterfly<T, M / 2, NVP>(x, lane);
   }
@@ -710,6 +755,15 @@ struct GridShape {
   static constexpr int NV = NE * 2 * NZ * 2;
 };
 
+// Bound by VALU issue: per triplet the distances, one cutoff product and an exp
+// per eta; per atom the radial lines and the reductions.  With the triplets left
+// out 500 of the FP32 kernel's 830 us remained at 65,000 atoms of 80 neighbours,
+// so the per-atom part counts as much as the triplets: reductions by cross-lane
+// moves (lane_xor) instead of LDS exchanges, a radial chunk of one cutoff group
+// without tests, two features a thread in the epilogue.  Together, per batch of
+// 67,647 atoms: FP64 1120 -> 974 us, FP32 413 -> 375; 65,000 atoms, FP32, without
+// forces to follow: 830 -> 750.  Every sum keeps its order, and FP32 features
+// their bits: the surrogate rounds them to BF16.
 template <typename T, int NZ, int W, bool Z16, bool FG>
 __global__ __launch_bounds__(W > 4 ? 64 * W : 256) void k_desc_fwd_grid(int N, const int *__restrict__ species,
                                                        const double *__restrict__ wz, NeighborBufs nb,
@@ -749,16 +803,31 @@ __global__ __launch_bounds__(W > 4 ? 64 * W : 256) void k_desc_fwd_grid(int N, c
     T acc[2 * RCH];
 #pragma unroll
     for (int l = 0; l < 2 * RCH; ++l) acc[l] = T(0);
-    for (int a = lane; a < K; a += 64) {
-      const T r = s_d[4 * a + 3], w = s_rw[2 * a + 1];
+    if (c0 + RCH <= sf.n_rad && sf.rad_g >= 0) {
+      // a whole chunk of one cutoff group: no test per line, the tables read
+      // in wide scalar loads and the cutoff once per neighbour
+      for (int a = lane; a < K; a += 64) {
+        const T r = s_d[4 * a + 3], w = s_rw[2 * a + 1], fc = s_fc[sf.rad_g * KP + a];
 #pragma unroll
-      for (int l = 0; l < RCH; ++l) {
-        const int s = c0 + l;
-        if (s < sf.n_rad) {
-          const T dr = r - rad_table<T>(sf.rad_rs, sf.rad_rs32, s);
-          const T t = Math<T>::ex(-rad_table<T>(sf.rad_a, sf.rad_a32, s) * dr * dr) * s_fc[sf.rad_group[s] * KP + a];
+        for (int l = 0; l < RCH; ++l) {
+          const T dr = r - rad_table<T>(sf.rad_rs, sf.rad_rs32, c0 + l);
+          const T t = Math<T>::ex(-rad_table<T>(sf.rad_a, sf.rad_a32, c0 + l) * dr * dr) * fc;
           acc[l] += t;
           acc[RCH + l] += t * w;
+        }
+      }
+    } else {
+      for (int a = lane; a < K; a += 64) {
+        const T r = s_d[4 * a + 3], w = s_rw[2 * a + 1];
+#pragma unroll
+        for (int l = 0; l < RCH; ++l) {
+          const int s = c0 + l;
+          if (s < sf.n_rad) {
+            const T dr = r - rad_table<T>(sf.rad_rs, sf.rad_rs32, s);
+            const T t = Math<T>::ex(-rad_table<T>(sf.rad_a, sf.rad_a32, s) * dr * dr) * s_fc[sf.rad_group[s] * KP + a];
+            acc[l] += t;
+            acc[RCH + l] += t * w;
+          }
         }
       }
     }
@@ -834,30 +903,7 @@ __global__ __launch_bounds__(W > 4 ? 64 * W : 256) void k_desc_fwd_grid(int N, c
     __syncthreads();
   }
 
-  // epilogue
-  double xn = 0.0;
-  const size_t row = (size_t)i * Dp;
-  for (int d = tid; d < Dp; d += 64 * W) {
-    const T x = s_feat[d];
-    if (out.x64) out.x64[row + d] = (double)x;
-    if (out.x32) out.x32[row + d] = (float)x;
-    const double xt = (double)x * theta_inv[d] - mu[d];
-    xn += xt * xt;
-    if (out.xt64) out.xt64[row + d] = xt;
-    if (out.xt32) out.xt32[row + d] = (float)xt;
-    if (split_mode == 1) {
-      const double xc = fp16_operand(xt);
-      const _Float16 hi = (_Float16)xc;
-      const _Float16 lo = (_Float16)(xc - (double)hi);
-      out.xt_hi[row + d] = __builtin_bit_cast(uint16_t, hi);
-      out.xt_lo[row + d] = __builtin_bit_cast(uint16_t, lo);
-    } else if (split_mode == 2) {
-      const __bf16 hi = (__bf16)(float)xt;
-      const __bf16 lo = (__bf16)(float)(xt - (double)(float)hi);
-      out.xt_hi[row + d] = __builtin_bit_cast(uint16_t, hi);
-      out.xt_lo[row + d] = __builtin_bit_cast(uint16_t, lo);
-    }
-  }
+  double xn = write_features<T, W>(s_feat, (size_t)i * Dp, Dp, tid, theta_inv, mu, split_mode, out);
   xn = wave_sum(xn);
   if (lane == 0) s_xn[wv] = xn;
   __syncthreads();

@@ -50,6 +50,7 @@ FORMS = {
     "eta9_zeta2": grid_sf(9, (2, 4)),
     "eta4_two_radial_cutoffs": grid_sf(4, (1, 2, 4, 8), rad_cuts=(6.0, 4.5)),
     "radial_only_wide": grid_sf(1, (1,), n_rad=37),
+    "radial_whole_chunk": grid_sf(2, (1, 4), n_rad=16),
     "no_grid": ring_sf(),
 }
 
