@@ -934,9 +934,12 @@ static int run_neighbors(Ctx &c, int flags, Bufs &b) {
   // built by the same wavefronts as the neighbour lists
   TripletBufs &tb = b.tb;
   tb.tcap = c.tcap;
-  if ((rc = c.get("trip_list", (size_t)c.N * c.tcap, &tb.list)) || (rc = c.get("trip_count", c.N, &tb.count)) ||
-      (rc = c.get("trip_raw", c.N, &tb.raw)))
+  tb.narrow = c.kcap <= kNarrowSlots;
+  unsigned char *list;
+  if ((rc = c.get("trip_list", (size_t)c.N * c.tcap * (tb.narrow ? 2 : 4), &list)) ||
+      (rc = c.get("trip_count", c.N, &tb.count)) || (rc = c.get("trip_raw", c.N, &tb.raw)))
     return rc;
+  tb.list = list;
   const bool ang = c.m->sf.n_ang > 0;
   GAPX_HIP(launch_build_neighbors(c.stream, c.N, d_astruct, d_sp, c.rcut, nb, c.m->sf.rc_max_ang, ang ? &tb : nullptr));
   if (!ang) {
@@ -1955,9 +1958,11 @@ static int ctx_car2acsf(Ctx &c, int na, int max_nb, int nf, const double *pos, c
   GAPX_HIP(launch_fill_int(c.stream, stats, 8, 0));
   // triplet lists: at most K (K - 1) / 2 pairs per atom, so no capacity retry
   tb.tcap = round_up(std::max(64, kmax * (kmax - 1) / 2), 64);
-  if ((rc = c.get("trip_list", (size_t)N * tb.tcap, &tb.list)) || (rc = c.get("trip_count", N, &tb.count)) ||
+  uint32_t *list;
+  if ((rc = c.get("trip_list", (size_t)N * tb.tcap, &list)) || (rc = c.get("trip_count", N, &tb.count)) ||
       (rc = c.get("trip_raw", N, &tb.raw)))
     return rc;
+  tb.list = list;
   if (m.sf.n_ang > 0)
     GAPX_HIP(launch_triplets_from_slots(c.stream, N, nb, m.sf.rc_max_ang, tb));
   else

@@ -359,13 +359,31 @@ __device__ __forceinline__ void stage_neighbours(const NeighborBufs &nb, const d
   }
 }
 
+// An atom's triplet list; an entry q is the pair (q & mask, q >> shift).
+struct TripletList {
+  const void *list;
+  int narrow;            // 16-bit entries
+  uint32_t mask, shift;
+  __device__ __forceinline__ TripletList(const TripletBufs &tb, int i)
+      : list(tb.narrow ? (const void *)((const uint16_t *)tb.list + (size_t)i * tb.tcap)
+                       : (const void *)((const uint32_t *)tb.list + (size_t)i * tb.tcap)),
+        narrow(tb.narrow), mask(tb.narrow ? 0xffu : 0xffffu), shift(tb.narrow ? 8u : 16u) {}
+};
+
 // Triplet indices of wave steps t, t + stride, .. (4 steps) for one lane; the
 // loads are issued together, one iteration ahead of their use, so a wave
 // waits for global memory once per four steps at most.  Inactive entries
 // point at neighbours 0 and 1 (valid whenever the list is not empty).
-__device__ __forceinline__ void load_q4(const uint32_t *tl, int nt, int t, int stride, uint32_t (&q)[4]) {
+__device__ __forceinline__ void load_q4(const TripletList &tl, int nt, int t, int stride, uint32_t (&q)[4]) {
+  if (tl.narrow) {
+    const uint16_t *p = (const uint16_t *)tl.list;
 #pragma unroll
-  for (int u = 0; u < 4; ++u) q[u] = (t + u * stride < nt) ? tl[t + u * stride] : (1u << 16);
+    for (int u = 0; u < 4; ++u) q[u] = (t + u * stride < nt) ? p[t + u * stride] : (1u << 8);
+  } else {
+    const uint32_t *p = (const uint32_t *)tl.list;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) q[u] = (t + u * stride < nt) ? p[t + u * stride] : (1u << 16);
+  }
 }
 
 // Front of the queue, the rest moved up (static register indices: the step's
@@ -384,10 +402,11 @@ __device__ __forceinline__ uint32_t pop_q4(uint32_t (&q)[4]) {
 // forward
 // ---------------------------------------------------------------------------
 template <typename T, int NCH>
-__device__ __forceinline__ void ang_fwd_term(uint32_t q, bool active, int c0, const SFDev &sf, const T *s_d,
+__device__ __forceinline__ void ang_fwd_term(const TripletList &tl, uint32_t q, bool active, int c0,
+                                             const SFDev &sf, const T *s_d,
                                              const T *s_rw, const T *s_fc, int KP, T (&acc)[NCH],
                                              T (&accw)[NCH]) {
-  const int a = q & 0xffff, b = q >> 16;
+  const int a = q & tl.mask, b = q >> tl.shift;
   const T ax = s_d[4 * a], ay = s_d[4 * a + 1], az = s_d[4 * a + 2], ra = s_d[4 * a + 3];
   const T bx = s_d[4 * b], by = s_d[4 * b + 1], bz = s_d[4 * b + 2], rb = s_d[4 * b + 3];
   const T ex = bx - ax, ey = by - ay, ez = bz - az;
@@ -508,7 +527,7 @@ __global__ __launch_bounds__(W > 4 ? 64 * W : 256) void k_desc_fwd(int N, const 
   }
 
   // angular lines, NCH at a time, over the atom's triplet list
-  const uint32_t *tl = tb.list + (size_t)i * tb.tcap;
+  const TripletList tl(tb, i);
   const int nt = tb.count[i];
   for (int c0 = 0; c0 < sf.n_ang; c0 += NCH) {
     T acc[NCH], accw[NCH];
@@ -522,7 +541,7 @@ __global__ __launch_bounds__(W > 4 ? 64 * W : 256) void k_desc_fwd(int N, const 
 #pragma unroll 1
       for (int u = 0; u < 4; ++u) {
         const uint32_t q = pop_q4(qc);
-        ang_fwd_term<T, NCH>(q, t0 + u * ST + lane < nt, c0, sf, s_d, s_rw, s_fc, KP, acc, accw);
+        ang_fwd_term<T, NCH>(tl, q, t0 + u * ST + lane < nt, c0, sf, s_d, s_rw, s_fc, KP, acc, accw);
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) qc[u] = qn[u];
@@ -837,7 +856,7 @@ __global__ __launch_bounds__(W > 4 ? 64 * W : 256) void k_desc_fwd_grid(int N, c
   }
 
   // angular lines in grid form, NE etas per pass
-  const uint32_t *tl = tb.list + (size_t)i * tb.tcap;
+  const TripletList tl(tb, i);
   const int nt = tb.count[i];
   const int g = sf.g_ang;
   const T rc = (T)sf.group_rc[g];
@@ -859,7 +878,7 @@ __global__ __launch_bounds__(W > 4 ? 64 * W : 256) void k_desc_fwd_grid(int N, c
       for (int u = 0; u < 4; ++u) {
         const bool act = t00 + u * ST + lane < nt;
         const uint32_t q = pop_q4(qc);
-        const int a = q & 0xffff, b = q >> 16;
+        const int a = q & tl.mask, b = q >> tl.shift;
         const T ax = s_d[4 * a], ay = s_d[4 * a + 1], az = s_d[4 * a + 2], ra = s_d[4 * a + 3];
         const T bx = s_d[4 * b], by = s_d[4 * b + 1], bz = s_d[4 * b + 2], rb = s_d[4 * b + 3];
         const T ex = bx - ax, ey = by - ay, ez = bz - az;
@@ -1024,13 +1043,14 @@ struct EtaRegs<double, ES> {
 };
 
 template <typename T, int NZ, bool Z16, int ES>
-__device__ __forceinline__ void ang_bwd_grid(uint32_t q, bool active, const SFDev &sf, const T *s_d, const T *s_rw,
+__device__ __forceinline__ void ang_bwd_grid(const TripletList &tl, uint32_t q, bool active,
+                                             const SFDev &sf, const T *s_d, const T *s_rw,
                                              const T *s_fd, const T *s_er, const EtaRegs<T, ES> &er,
                                              const T (&ceta)[4 * ES + 1], const T (&eta)[4 * ES + 1], int KP, T rc,
                                              T pirc, double *s_T, double *s_F) {
   // idle lanes work on neighbours 0 and 1 (the products need every lane) and
   // add nothing at the end
-  const int a = q & 0xffff, b = q >> 16;
+  const int a = q & tl.mask, b = q >> tl.shift;
   const T ax = s_d[4 * a], ay = s_d[4 * a + 1], az = s_d[4 * a + 2], ra = s_d[4 * a + 3];
   const T bx = s_d[4 * b], by = s_d[4 * b + 1], bz = s_d[4 * b + 2], rb = s_d[4 * b + 3];
   typedef typename Pair<T>::type P2;
@@ -1126,11 +1146,12 @@ __device__ __forceinline__ void ang_bwd_grid(uint32_t q, bool active, const SFDe
 // backward
 // ---------------------------------------------------------------------------
 template <typename T>
-__device__ __forceinline__ void ang_bwd_term(uint32_t q, bool active, const SFDev &sf, const T *s_d,
+__device__ __forceinline__ void ang_bwd_term(const TripletList &tl, uint32_t q, bool active,
+                                             const SFDev &sf, const T *s_d,
                                              const T *s_rw, const T *s_fd, const T *s_gA, const T *s_gW, int KP,
                                              double *s_T, double *s_F) {
   if (!active) return;
-  const int a = q & 0xffff, b = q >> 16;
+  const int a = q & tl.mask, b = q >> tl.shift;
   const T ax = s_d[4 * a], ay = s_d[4 * a + 1], az = s_d[4 * a + 2], ra = s_d[4 * a + 3];
   const T bx = s_d[4 * b], by = s_d[4 * b + 1], bz = s_d[4 * b + 2], rb = s_d[4 * b + 3];
   const T ex = bx - ax, ey = by - ay, ez = bz - az;
@@ -1391,7 +1412,7 @@ __global__ __launch_bounds__(W > 4 ? 64 * W : 256, 2) void k_desc_bwd(int N, con
   __syncthreads();
 
   if (sf.n_ang > 0) {
-    const uint32_t *tl = tb.list + (size_t)i * tb.tcap;
+    const TripletList tl(tb, i);
     const int nt = tb.count[i];
     const T rcA = (T)sf.group_rc[sf.g_ang], pirc = (T)sf.group_pirc[sf.g_ang];
     constexpr int ST = 64 * W;
@@ -1405,10 +1426,10 @@ __global__ __launch_bounds__(W > 4 ? 64 * W : 256, 2) void k_desc_bwd(int N, con
         const bool act = t0 + u * ST + lane < nt;
         const uint32_t q = pop_q4(qc);
         if constexpr (GNZ > 0)
-          ang_bwd_grid<T, GNZ, Z16, ES>(q, act, sf, s_d, s_rw, s_fd, s_er, er, ceta, eta, KP, rcA, pirc,
+          ang_bwd_grid<T, GNZ, Z16, ES>(tl, q, act, sf, s_d, s_rw, s_fd, s_er, er, ceta, eta, KP, rcA, pirc,
                                         s_T + wv * KP, s_F + 3 * wv * KP);
         else
-          ang_bwd_term<T>(q, act, sf, s_d, s_rw, s_fd, s_gA, s_gW, KP, s_T + wv * KP, s_F + 3 * wv * KP);
+          ang_bwd_term<T>(tl, q, act, sf, s_d, s_rw, s_fd, s_gA, s_gW, KP, s_T + wv * KP, s_F + 3 * wv * KP);
       }
 #pragma unroll
       for (int u = 0; u < 4; ++u) qc[u] = qn[u];

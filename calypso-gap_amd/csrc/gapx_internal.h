@@ -192,11 +192,16 @@ struct DescOut {
   double *xn;           // [N] |xt|^2 (FP64)
 };
 
+// Longest list whose triplets are kept in 16 bits (8 per neighbour).
+constexpr int kNarrowSlots = 256;
+
 // Per-atom triplet lists: neighbour pairs (a, b), a < b, with r_a, r_b and
-// r_ab within the largest angular cutoff, packed a | b << 16 at i * tcap.
+// r_ab within the largest angular cutoff, at i * tcap: packed a | b << 16 in 32
+// bits, or, where every list has at most 256 slots (narrow), a | b << 8 in 16.
 struct TripletBufs {
   int tcap;
-  uint32_t *list;       // [N*tcap]
+  int narrow;
+  void *list;           // [N*tcap] uint16_t (narrow) or uint32_t
   int *count;           // [N] kept triplets (<= tcap)
   int *raw;             // [N] triplet count before the tcap clamp
 };

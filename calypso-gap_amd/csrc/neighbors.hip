@@ -319,8 +319,8 @@ __device__ __forceinline__ int sext5(uint32_t v) { return (int)((v & 31u) ^ 16u)
 // Triplet lists, from the neighbour records the building wave just staged in
 // LDS.  Pairs (a, b), a < b, with r_a, r_b, r_ab all within the largest
 // angular cutoff are appended (ballot + prefix count) to the atom's list at
-// i * tcap, packed as a | b << 16, in diagonal order: the pairs with b - a = d
-// form a run of K - d entries.  Runs d and K - d together hold K entries, so
+// i * tcap, packed as a | b << 16 or a | b << 8, in diagonal order: the pairs
+// with b - a = d form a run of K - d entries.  Runs d and K - d together hold K entries, so
 // one wave step takes both (full lanes for K <= 64).  Consecutive entries of
 // a run have distinct a and distinct b, so the backward pass's LDS atomics on
 // per-neighbour accumulators rarely collide within one instruction.  Entry c
@@ -347,54 +347,79 @@ __host__ __device__ constexpr size_t trip_lds_records(int kcap) {
   return (size_t)std::max(kcap, std::min(kcap, 256) + std::min(kcap, 256) / 2);
 }
 
+// NARROW: 16-bit entries (lists of at most kNarrowSlots slots).  Half the bytes
+// of the list, which the wave's appends and the descriptor kernels' reads both
+// pay for: 130 M triplets took 140 of k_build's 506 us to store in 32 bits.
+template <bool NARROW>
 __device__ __forceinline__ void triplets_from_lds(int i, int K, float4 *s_p, double rcA, const TripletBufs &tb,
                                                   int lane) {
   constexpr int kOwn = 4;  // register-held record chunks: K <= 64 kOwn
+  constexpr int SH = NARROW ? 8 : 16;
+  typedef typename std::conditional<NARROW, uint16_t, uint32_t>::type Entry;
   K = __builtin_amdgcn_readfirstlane(K);
   const float rc = trip_rc(rcA);
   const float rc2 = rc * rc;
-  uint32_t *out = tb.list + (size_t)i * tb.tcap;
+  Entry *out = (Entry *)tb.list + (size_t)i * tb.tcap;
   int count = 0;
   // pairs of the step whose lanes pass `ok`, appended after `count` entries
   auto emit = [&](bool ok, uint32_t pair) {
     const unsigned long long m = __ballot(ok);
     const unsigned pre = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
-    if (ok && (int)pre < tb.tcap - count) out[count + pre] = pair;
+    if (ok && (int)pre < tb.tcap - count) out[count + pre] = (Entry)pair;
     count += __popcll(m);
   };
   if (K <= 64 * kOwn) {
     for (int t = lane; t < K / 2; t += 64) s_p[K + t] = s_p[t];
     __syncthreads();
     const int KX = K + K / 2;  // records readable at c + d
-    float4 own[kOwn];
-    uint32_t self[kOwn];  // c | c << 16
+    // Q chunks of 64 neighbours: the records of U steps are read together, so
+    // a wave waits for LDS once per U Q entries rather than for each
+    auto runs = [&](auto chunks, auto steps) {
+      constexpr int Q = decltype(chunks)::value, U = decltype(steps)::value;
+      float4 own[Q];
+      uint32_t self[Q];  // c | c << SH
 #pragma unroll
-    for (int q = 0; q < kOwn; ++q) {
-      const int c = 64 * q + lane;
-      own[q] = s_p[min(c, max(K - 1, 0))];
-      if (c >= K) own[q].x = __builtin_nanf("");  // idle lanes fail every test
-      self[q] = (uint32_t)c | ((uint32_t)c << 16);
-    }
-    // one step: run d1 (K - d1 pairs) and run K - d1 (d1 pairs), or, when the
-    // two are the same run (2 d1 = K), its n = K - d1 pairs only
-    auto step = [&](int d1, int n, auto whole) {
-      const int n1 = K - d1;
-      const uint32_t lo = (uint32_t)(d1 - K), hi = (uint32_t)d1 << 16;
-#pragma unroll
-      for (int q = 0; q < kOwn; ++q) {
-        if (64 * q >= n) break;
+      for (int q = 0; q < Q; ++q) {
         const int c = 64 * q + lane;
-        const float4 pp = s_p[min(c + d1, KX - 1)];
-        const float ex = pp.x - own[q].x, ey = pp.y - own[q].y, ez = pp.z - own[q].z;
-        bool ok = ex * ex + ey * ey + ez * ez <= rc2;
-        if (!decltype(whole)::value) ok = ok && c < n;
-        // run d1: (c, c + d1); run K - d1: (c + d1 - K, c)
-        emit(ok, self[q] + (c < n1 ? hi : lo));
+        own[q] = s_p[min(c, max(K - 1, 0))];
+        if (c >= K) own[q].x = __builtin_nanf("");  // idle lanes fail every test
+        self[q] = (uint32_t)c | ((uint32_t)c << SH);
       }
+      // one step: run d1 (K - d1 pairs) and run K - d1 (d1 pairs), or, when the
+      // two are the same run (2 d1 = K), its n = K - d1 pairs only
+      auto batch = [&](int d0, int live) {
+        float4 pp[U][Q];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int q = 0; q < Q; ++q) pp[u][q] = s_p[min(64 * q + lane + d0 + u, KX - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          if (u >= live) break;
+          const int d1 = d0 + u, n1 = K - d1, n = 2 * d1 == K ? n1 : K;
+          const uint32_t lo = (uint32_t)(d1 - K), hi = (uint32_t)d1 << SH;
+#pragma unroll
+          for (int q = 0; q < Q; ++q) {
+            const int c = 64 * q + lane;
+            const float ex = pp[u][q].x - own[q].x, ey = pp[u][q].y - own[q].y, ez = pp[u][q].z - own[q].z;
+            const bool ok = (ex * ex + ey * ey + ez * ez <= rc2) & (c < n);
+            // run d1: (c, c + d1); run K - d1: (c + d1 - K, c)
+            emit(ok, self[q] + (c < n1 ? hi : lo));
+          }
+        }
+      };
+      const int last = K / 2;  // steps d1 = 1 .. K / 2
+      for (int d0 = 1; d0 <= last; d0 += U) batch(d0, min(U, last - d0 + 1));
     };
-    int d1 = 1;
-    for (; 2 * d1 < K; ++d1) step(d1, K, std::true_type{});
-    if (2 * d1 == K) step(d1, K - d1, std::false_type{});
+    typedef std::integral_constant<int, 1> C1;
+    typedef std::integral_constant<int, 2> C2;
+    typedef std::integral_constant<int, 4> C4;
+    if (K <= 64)
+      runs(C1{}, C4{});
+    else if (K <= 128)
+      runs(C2{}, C2{});
+    else
+      runs(C4{}, C1{});
   } else {
     for (int d1 = 1; 2 * d1 <= K; ++d1) {
       // run d1 (K - d1 pairs), then run d2 = K - d1 (d1 pairs) unless it is d1
@@ -409,7 +434,7 @@ __device__ __forceinline__ void triplets_from_lds(int i, int K, float4 *s_p, dou
         const bool live = c < n;
         const float4 pa = s_p[live ? a : 0], pb = s_p[live ? b : 0];
         const float ex = pb.x - pa.x, ey = pb.y - pa.y, ez = pb.z - pa.z;
-        emit(live & (ex * ex + ey * ey + ez * ez <= rc2), (uint32_t)a | ((uint32_t)b << 16));
+        emit(live & (ex * ex + ey * ey + ez * ez <= rc2), (uint32_t)a | ((uint32_t)b << SH));
       }
     }
   }
@@ -419,23 +444,53 @@ __device__ __forceinline__ void triplets_from_lds(int i, int K, float4 *s_p, dou
   }
 }
 
+// A bin image that holds atoms: its first atom's slot less the candidates
+// before it, its lattice translation (three components of -64 .. 64 in bytes)
+// and that translation's vector.
+struct ImageRec {
+  int first, t;
+  double sx, sy, sz;
+};
+
+// Inclusive prefix sum over the wave by row shifts and row broadcasts.
+__device__ __forceinline__ int wave_prefix(int v) {
+#define GAPX_SCAN(ctrl, rows) v += __builtin_amdgcn_update_dpp(0, v, ctrl, rows, 0xf, false)
+  GAPX_SCAN(0x111, 0xf);  // row_shr:1
+  GAPX_SCAN(0x112, 0xf);  // row_shr:2
+  GAPX_SCAN(0x114, 0xf);  // row_shr:4
+  GAPX_SCAN(0x118, 0xf);  // row_shr:8
+  GAPX_SCAN(0x142, 0xa);  // row_bcast:15 into rows 1 and 3
+  GAPX_SCAN(0x143, 0xc);  // row_bcast:31 into rows 2 and 3
+#undef GAPX_SCAN
+  return v;
+}
+
 // One wavefront per centre atom.  The (2S+1)^3 bin images are taken 64 at a
 // time, one per lane (bin range and image shift); a wave prefix sum over the
 // bin sizes flattens their atoms into one candidate sequence, which the lanes
-// then test 64 at a time, each finding its image by a binary search over the
-// prefix sums.  Accepted pairs are appended with ballot + prefix count, so the
-// list order is image order, then index order inside the bin (deterministic).
+// then test 64 at a time, each finding its image from a bit mask of the places
+// where images start.  Accepted pairs are appended with ballot + prefix count, so
+// the list order is image order, then index order inside the bin (deterministic).
 // Slots live at i * kcap + a; counts above kcap are recorded, not written.
 // With TRIP the wave also keeps each kept neighbour's (dx, dy, dz, r) in LDS
 // (FP32) and builds the atom's triplet list from there (triplets_from_lds).
+// Bound by VALU issue and the lists' stores; of 506 us for 143,416 atoms of 63
+// neighbours the triplets took 220 (140 of them stores), the candidates 214, the
+// set-up 70.  16-bit triplets, LDS reads a batch of runs ahead, image records in
+// LDS instead of shuffles (a binary search of six and five fetches per
+// candidate) and a prefix sum by row shifts: 506 -> 433 us.
 template <bool TRIP>
 __global__ __launch_bounds__(64) void k_build(int N, const int *__restrict__ atom_struct,
                                               const StructParams *__restrict__ sp, double rcut, NeighborBufs nb,
                                               double rcA, TripletBufs tb) {
   extern __shared__ __align__(16) unsigned char smem[];
   float4 *s_p = (float4 *)smem;  // [trip_lds_records(kcap)] with TRIP
+  __shared__ ImageRec s_rec[64];
+  __shared__ int s_flag[64];
   const int i = blockIdx.x, lane = threadIdx.x;
   if (i >= N) return;
+  s_flag[lane] = 0;
+  int mark = 0;
   const StructParams &P = sp[atom_struct[i]];
   const int b = nb.atom_bin[i] - P.bin_base;
   const int bi2 = b % P.nb[2], bi1 = (b / P.nb[2]) % P.nb[1], bi0 = b / (P.nb[1] * P.nb[2]);
@@ -495,22 +550,40 @@ __global__ __launch_bounds__(64) void k_build(int N, const int *__restrict__ ato
         n = nb.bin_start[bin + 1] - lo;
       }
     }
-    int incl = n;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += v;
+    const int incl = wave_prefix(n);
+    const int total = __builtin_amdgcn_readlane(incl, 63);
+    const int excl = incl - n;
+    // the group's bins that hold atoms, compacted in image order: candidate c of
+    // a bin sits at slot first + c, its atoms are shifted by the lattice vector
+    const unsigned long long held = __ballot(n > 0);
+    const unsigned below =
+        __builtin_amdgcn_mbcnt_hi((unsigned)(held >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)held, 0u));
+    if (n > 0) {
+      ImageRec rec;
+      rec.first = lo - excl;
+      rec.t = (t0 + 64) | ((t1 + 64) << 8) | ((t2 + 64) << 16);
+      rec.sx = t0 * P.L[0] + t1 * P.L[3] + t2 * P.L[6];
+      rec.sy = t0 * P.L[1] + t1 * P.L[4] + t2 * P.L[7];
+      rec.sz = t0 * P.L[2] + t1 * P.L[5] + t2 * P.L[8];
+      s_rec[below] = rec;
     }
-    const int total = __shfl(incl, 63, 64);
-    const int first = lo - (incl - n);  // candidate c of this image sits at slot first + c
     for (int c0 = 0; c0 < total; c0 += 64) {
       const int c = c0 + lane;
-      int src = 0;  // number of images whose prefix ends at or before c
-#pragma unroll
-      for (int step = 32; step > 0; step >>= 1)
-        if (__shfl(incl, src + step - 1, 64) <= c) src += step;
-      const int q = __shfl(first, src, 64) + c;
-      const int T0 = __shfl(t0, src, 64), T1 = __shfl(t1, src, 64), T2 = __shfl(t2, src, 64);
+      // a lane's bin: the bins before this batch plus those that start at or
+      // before the lane, which mark their first candidate's place
+      ++mark;
+      const int at = excl - c0;
+      if (n > 0 && at >= 0 && at < 64) s_flag[at] = mark;
+      __syncthreads();
+      const unsigned long long starts = __ballot(s_flag[lane] == mark);
+      const int before = __popcll(__ballot(n > 0 && at < 0));
+      const unsigned upto = __builtin_amdgcn_mbcnt_hi((unsigned)(starts >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo((unsigned)starts, 0u)) +
+                            (unsigned)((starts >> lane) & 1ull);
+      const ImageRec rec = s_rec[max(before + (int)upto - 1, 0)];
+      __syncthreads();  // read before the next batch's marks
+      const int q = rec.first + c;
+      const int T0 = (rec.t & 255) - 64, T1 = ((rec.t >> 8) & 255) - 64, T2 = (rec.t >> 16) - 64;
       bool ok = false;
       int4 inf = make_int4(0, 0, 0, 0);
       double dx = 0, dy = 0, dz = 0, r = 0;
@@ -518,12 +591,9 @@ __global__ __launch_bounds__(64) void k_build(int N, const int *__restrict__ ato
         inf = sinfo[q];
         const double2 pxy = sp2[2 * (size_t)q], pz = sp2[2 * (size_t)q + 1];
         if (!(T0 == 0 && T1 == 0 && T2 == 0 && inf.x == i)) {
-          const double sx = T0 * P.L[0] + T1 * P.L[3] + T2 * P.L[6];
-          const double sy = T0 * P.L[1] + T1 * P.L[4] + T2 * P.L[7];
-          const double sz = T0 * P.L[2] + T1 * P.L[5] + T2 * P.L[8];
-          dx = pxy.x + sx - xi;
-          dy = pxy.y + sy - yi;
-          dz = pz.x + sz - zi;
+          dx = pxy.x + rec.sx - xi;
+          dy = pxy.y + rec.sy - yi;
+          dz = pz.x + rec.sz - zi;
           r = sqrt(dx * dx + dy * dy + dz * dz);
           ok = !(r > rcut);
         }
@@ -552,7 +622,10 @@ __global__ __launch_bounds__(64) void k_build(int N, const int *__restrict__ ato
   }
   if (TRIP) {
     __syncthreads();
-    triplets_from_lds(i, min(count, nb.kcap), s_p, rcA, tb, lane);
+    if (tb.narrow)
+      triplets_from_lds<true>(i, min(count, nb.kcap), s_p, rcA, tb, lane);
+    else
+      triplets_from_lds<false>(i, min(count, nb.kcap), s_p, rcA, tb, lane);
   }
 }
 
@@ -571,7 +644,7 @@ __global__ __launch_bounds__(64) void k_triplets_from_slots(int N, NeighborBufs 
     s_p[a] = trip_record(d[0], d[1], d[2], d[3], trip_rc(rcA));
   }
   __syncthreads();
-  triplets_from_lds(i, K, s_p, rcA, tb, lane);
+  triplets_from_lds<false>(i, K, s_p, rcA, tb, lane);
 }
 
 // |pos_i - (pos_j + n1 L1 + n2 L2 + n3 L3)| in the order of operations of
