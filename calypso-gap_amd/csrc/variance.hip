@@ -14,7 +14,8 @@
 //   k_var_kernel    K = exp(-(|xt_i|^2 + |mt_k|^2 - 2 xt_i . mt_k) / 2) for a
 //                   64-row x 64-point tile per workgroup, the points staged in
 //                   LDS 32 features at a time,
-//   k_var_quad      U = K Q for a 64 x 64 tile per workgroup (K and Q staged
+//   k_var_quad      U = K Q for a 64 x 64 tile per workgroup, or 128 x 128
+//                   (k_var_quad128) where those fill the chip (K and Q staged
 //                   in LDS 32 points at a time), contracted with K in the
 //                   epilogue: partial[column tile][i] = sum over the tile's
 //                   columns c of U_ic K_ic, so U never reaches memory,
@@ -150,6 +151,93 @@ __global__ __launch_bounds__(256) void k_var_quad(int N, int r0, int Mp, const d
   }
 }
 
+// The same for 128 x 128 tiles: wave (w / 2, w % 2) holds a 64 x 64 quarter in
+// 16 accumulators, so a step of 4 points reads 8 operands from LDS for 16
+// products (5 for 4 above); the next 16 points travel to registers while the
+// current ones multiply, and go to the other LDS buffer behind them, with one
+// barrier per chunk: 48 -> 64 TF/s (2048 atoms, 4032 points, 1168 -> 1063 us; the
+// matrix cores 93 % busy at the 2.1 GHz the card runs here).  Rows of A are 18 doubles apart, rows of B 144: operand
+// reads of 32 lanes fall on 64 different banks.  A tile's edge rows (rows is a multiple of 64) and columns repeat the
+// last one and are not stored; the partials are those of k_var_quad, in its
+// order of operations.
+constexpr int kQC = 16, kQA = kQC + 2, kQB = 128 + 16;
+
+__global__ __launch_bounds__(256, 2) void k_var_quad128(int N, int r0, int rows, int Mp, const double *__restrict__ K,
+                                                        const double *__restrict__ Q, double *__restrict__ partial) {
+  __shared__ __align__(16) double s_a[2][128 * kQA];
+  __shared__ __align__(16) double s_b[2][kQC * kQB];
+  const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int l16 = lane & 15, lq = lane >> 4;
+  const int wr = wv >> 1, wc = wv & 1;
+  const int rb = blockIdx.x * 128, c0 = blockIdx.y * 128;
+  typedef double v4d __attribute__((ext_vector_type(4)));
+  v4d acc[4][4];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int b = 0; b < 4; ++b) acc[a][b] = v4d{0, 0, 0, 0};
+  // pieces of two doubles, four of each tile per thread
+  const double *pa[4], *pq[4];
+  int oa[4], ob[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    const int e = tid + 256 * u;
+    const int ar = e / (kQC / 2), ac = 2 * (e % (kQC / 2));  // K tile: row ar, points ac, ac + 1
+    const int br = e / 64, bc = 2 * (e % 64);                // Q tile: point br, columns bc, bc + 1
+    pa[u] = K + (size_t)min(rb + ar, rows - 1) * Mp + ac;
+    pq[u] = Q + (size_t)br * Mp + min(c0 + bc, Mp - 2);
+    oa[u] = ar * kQA + ac;
+    ob[u] = br * kQB + bc;
+  }
+  typedef double v2d __attribute__((ext_vector_type(2)));
+  v2d va0, va1, va2, va3, vb0, vb1, vb2, vb3;  // named: an array of them went to scratch memory
+#define GAPX_FETCH(u, k) \
+  va##u = *(const v2d *)(pa[u] + (k)), vb##u = *(const v2d *)(pq[u] + (size_t)(k) * Mp)
+#define GAPX_PUT(u, buf) *(v2d *)(s_a[buf] + oa[u]) = va##u, *(v2d *)(s_b[buf] + ob[u]) = vb##u
+  GAPX_FETCH(0, 0), GAPX_FETCH(1, 0), GAPX_FETCH(2, 0), GAPX_FETCH(3, 0);
+  GAPX_PUT(0, 0), GAPX_PUT(1, 0), GAPX_PUT(2, 0), GAPX_PUT(3, 0);
+  __syncthreads();
+  int buf = 0;
+  for (int k0 = 0; k0 < Mp; k0 += kQC) {
+    const int kn = min(k0 + kQC, Mp - kQC);  // the last chunk once more at the end: no branch around live registers
+    GAPX_FETCH(0, kn), GAPX_FETCH(1, kn), GAPX_FETCH(2, kn), GAPX_FETCH(3, kn);
+    const double *la = s_a[buf] + (64 * wr + l16) * kQA + lq, *lb = s_b[buf] + lq * kQB + 64 * wc + l16;
+#pragma unroll
+    for (int t = 0; t < kQC / 4; ++t) {
+      double a[4], b[4];
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        a[x] = la[16 * x * kQA + 4 * t];
+        b[x] = lb[4 * t * kQB + 16 * x];
+      }
+#pragma unroll
+      for (int x = 0; x < 4; ++x)
+#pragma unroll
+        for (int y = 0; y < 4; ++y) acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[x], b[y], acc[x][y], 0, 0, 0);
+    }
+    GAPX_PUT(0, buf ^ 1), GAPX_PUT(1, buf ^ 1), GAPX_PUT(2, buf ^ 1), GAPX_PUT(3, buf ^ 1);
+    __syncthreads();
+    buf ^= 1;
+  }
+#undef GAPX_FETCH
+#undef GAPX_PUT
+  const int ct = 2 * blockIdx.y + wc, cc = 64 * ct;
+  if (cc >= Mp) return;
+#pragma unroll
+  for (int x = 0; x < 4; ++x)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int ib = rb + 64 * wr + 16 * x + lq + 4 * r;
+      if (ib >= rows) continue;  // the same for a whole 16-row block
+      double s = 0.0;
+#pragma unroll
+      for (int b = 0; b < 4; ++b) s += acc[x][b][r] * K[(size_t)ib * Mp + cc + 16 * b + l16];
+#pragma unroll
+      for (int o = 8; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+      if (l16 == 0 && r0 + ib < N) partial[(size_t)ct * N + r0 + ib] = s;
+    }
+}
+
 // sigma2_i = delta - sum over column tiles of the partials, in tile order.
 __global__ __launch_bounds__(256) void k_var_finish(int N, int ntiles, const double *__restrict__ partial,
                                                     double *__restrict__ sigma2) {
@@ -177,6 +265,17 @@ __global__ __launch_bounds__(256) void k_struct_mean(int nstruct, const StructPa
   if (t == 0) var[s] = n > 0 ? ((part[0] + part[1]) + (part[2] + part[3])) / n : 0.0;
 }
 
+// Which tile of the quadratic form.  A round of one tile on each of the 256 CUs
+// takes as long as 3.6 of the small tile's for the wide one (535 and 148 us at
+// 4032 points: the wide tile does four times the work), so the wide tile wins
+// where its rounds are full.  Small and wide, us a pass: 512 atoms 396 665, 700
+// 546 670, 1024 823 673, 1500 1004 1180, 2048 1299 1194, 2100 1463 1731, 4096
+// 2507 2314, 8192 5038 4500.
+bool wide_tiles(unsigned small, unsigned wide) {
+  const unsigned cu = 256;
+  return 18 * ((wide + cu - 1) / cu) < 5 * ((small + cu - 1) / cu);
+}
+
 }  // namespace
 
 int enqueue_variance(hipStream_t s, const VarianceArgs &v) {
@@ -201,7 +300,11 @@ int enqueue_variance(hipStream_t s, const VarianceArgs &v) {
       const dim3 grid(rows / 64, ntiles);
       k_var_kernel<<<grid, 256, 0, s>>>(v.N, r0, v.Dp, v.Mp, xt, v.xn, v.mt, v.mn, v.K);
       GAPX_HIP(hipGetLastError());
-      k_var_quad<<<grid, 256, 0, s>>>(v.N, r0, v.Mp, v.K, v.qmm, v.partial);
+      const dim3 wide((rows + 127) / 128, (v.Mp + 127) / 128);
+      if (wide_tiles(grid.x * grid.y, wide.x * wide.y))
+        k_var_quad128<<<wide, 256, 0, s>>>(v.N, r0, rows, v.Mp, v.K, v.qmm, v.partial);
+      else
+        k_var_quad<<<grid, 256, 0, s>>>(v.N, r0, v.Mp, v.K, v.qmm, v.partial);
       GAPX_HIP(hipGetLastError());
     }
     k_var_finish<<<(v.N + 255) / 256, 256, 0, s>>>(v.N, ntiles, v.partial, v.sigma2);
