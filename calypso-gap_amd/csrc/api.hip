@@ -1732,6 +1732,13 @@ static int ctx_relax_lbfgs(Ctx &c, int flags, int max_steps, double fmax, double
 // so the trajectory is the one every-step checking would give.
 static constexpr double kBoltzmannEv = 8.6173303e-5;  // eV/K, CODATA 2014 (ASE 3.18.1 units)
 static constexpr int kMdCheckEvery = 16;
+// Up to this many atoms in the largest structure all that lies between two
+// evaluations is one launch of one workgroup per structure, above it four (of
+// which the kick and the drift use one thread per atom).  Four and one, us a
+// step: 64 atoms 107 99, 512 134 125, 2048 221 212, 8192 554 547, 64 structures of
+// 128 atoms 454 441; a workgroup's pass over larger structures takes what the
+// three launches save.
+static constexpr int kMdTurnAtoms = 8192;
 
 static int ctx_md(Ctx &c, int flags, int nsteps, double dt, double temperature, double taut, int fixcm,
                   const double *masses, const double *momenta, double *log) {
@@ -1759,10 +1766,13 @@ static int ctx_md(Ctx &c, int flags, int nsteps, double dt, double temperature, 
   const MdParams mp{dt, temperature, taut, kBoltzmannEv, fixcm ? 1 : 0, 0};
   const StructParams *d_sp = c.d_sp;
   const int *d_as = c.d_astruct;
+  int largest = 0;
+  for (int s = 0; s < c.nstruct; ++s) largest = std::max(largest, c.sp[s].natoms);
+  const bool one_turn = largest <= kMdTurnAtoms;
   if ((rc = ctx_run(c, flags)) || (rc = ctx_settle(c))) return rc;
   trajectory_headroom(c);
-  if (dlog) GAPX_HIP(launch_md_log(c.stream, c.nstruct, d_sp, mass, p, c.d_force, c.d_ene,
-                                   mp.kB, dlog));
+  if (dlog)
+    GAPX_HIP(launch_md_turn(c.stream, c.nstruct, d_sp, mass, c.d_force, mp, false, false, c.d_ene, p, c.d_pos, dlog));
   int hs[8];
   for (int b0 = 0, redo = 0; b0 < nsteps;) {
     const int nb = std::min(kMdCheckEvery, nsteps - b0);
@@ -1775,15 +1785,24 @@ static int ctx_md(Ctx &c, int flags, int nsteps, double dt, double temperature, 
     int *sticky = c.ptr<int>("stats_acc") + 8;
     GAPX_HIP(launch_fill_int(c.stream, sticky, 8, 0));
     for (int step = b0; step < b0 + nb; ++step) {
-      double *x = c.d_pos, *f = c.d_force;
-      GAPX_HIP(launch_md_prepare(c.stream, c.nstruct, d_sp, mass, p, f, mp, coef));
-      GAPX_HIP(launch_md_drift(c.stream, c.N, d_as, mass, f, coef, dt, p, x));
+      if (!one_turn) {
+        GAPX_HIP(launch_md_prepare(c.stream, c.nstruct, d_sp, mass, p, c.d_force, mp, coef));
+        GAPX_HIP(launch_md_drift(c.stream, c.N, d_as, mass, c.d_force, coef, dt, p, c.d_pos));
+      } else if (step == b0) {
+        GAPX_HIP(launch_md_turn(c.stream, c.nstruct, d_sp, mass, c.d_force, mp, false, true, c.d_ene, p, c.d_pos,
+                                nullptr));
+      }
       if ((rc = ctx_run(c, flags))) return rc;
-      f = c.d_force;
-      GAPX_HIP(launch_md_kick(c.stream, c.N, f, 0.5 * dt, p));
-      if (dlog)
-        GAPX_HIP(launch_md_log(c.stream, c.nstruct, d_sp, mass, p, f, c.d_ene, mp.kB,
-                               dlog + 3 * (size_t)c.nstruct * (step + 1)));
+      double *entry = dlog ? dlog + 3 * (size_t)c.nstruct * (step + 1) : nullptr;
+      if (one_turn) {
+        GAPX_HIP(launch_md_turn(c.stream, c.nstruct, d_sp, mass, c.d_force, mp, true, step + 1 < b0 + nb, c.d_ene, p,
+                                c.d_pos, entry));
+      } else {
+        GAPX_HIP(launch_md_kick(c.stream, c.N, c.d_force, 0.5 * dt, p));
+        if (entry)
+          GAPX_HIP(launch_md_turn(c.stream, c.nstruct, d_sp, mass, c.d_force, mp, false, false, c.d_ene, p, c.d_pos,
+                                  entry));
+      }
     }
     sticky = c.ptr<int>("stats_acc") + 8;
     GAPX_HIP(hipMemcpyAsync(hs, sticky, sizeof hs, hipMemcpyDeviceToHost, c.stream));
