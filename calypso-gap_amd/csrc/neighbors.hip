@@ -203,6 +203,19 @@ __global__ __launch_bounds__(64) void k_rank_bins(int nbins, NeighborBufs nb) {
   }
 }
 
+// Inclusive prefix sum over the wave by row shifts and row broadcasts.
+__device__ __forceinline__ int wave_prefix(int v) {
+#define GAPX_SCAN(ctrl, rows) v += __builtin_amdgcn_update_dpp(0, v, ctrl, rows, 0xf, false)
+  GAPX_SCAN(0x111, 0xf);  // row_shr:1
+  GAPX_SCAN(0x112, 0xf);  // row_shr:2
+  GAPX_SCAN(0x114, 0xf);  // row_shr:4
+  GAPX_SCAN(0x118, 0xf);  // row_shr:8
+  GAPX_SCAN(0x142, 0xa);  // row_bcast:15 into rows 1 and 3
+  GAPX_SCAN(0x143, 0xc);  // row_bcast:31 into rows 2 and 3
+#undef GAPX_SCAN
+  return v;
+}
+
 // One workgroup per structure does the whole binning in LDS: wrap and bin
 // every atom, count per bin, exclusive scan, scatter, then order each bin's
 // atoms by index and write the bin-sorted records; workgroup 0 also clears
@@ -260,15 +273,12 @@ __global__ __launch_bounds__(1024) void k_bin_struct(const double *__restrict__ 
   const int per = (nbs + 1023) / 1024, lo = t * per, hi = min(nbs, lo + per);
   int sum = 0;
   for (int b = lo; b < hi; ++b) sum += s_cnt[b];
-  s_part[t] = sum;
+  // (within the wave by row shifts, then over the sixteen waves' totals)
+  const int incl = wave_prefix(sum);
+  if ((t & 63) == 63) s_part[t >> 6] = incl;
   __syncthreads();
-  for (int off = 1; off < 1024; off <<= 1) {
-    const int v = (t >= off) ? s_part[t - off] : 0;
-    __syncthreads();
-    s_part[t] += v;
-    __syncthreads();
-  }
-  int run = s_part[t] - sum;
+  const int tot = wave_prefix((t & 63) < 16 ? s_part[t & 63] : 0);  // of waves 0 .. lane
+  int run = incl - sum + (t >= 64 ? __shfl(tot, max((t >> 6) - 1, 0), 64) : 0);
   for (int b = lo; b < hi; ++b) {
     const int v = s_cnt[b];
     s_cnt[b] = run;
@@ -350,9 +360,11 @@ __host__ __device__ constexpr size_t trip_lds_records(int kcap) {
 // NARROW: 16-bit entries (lists of at most kNarrowSlots slots).  Half the bytes
 // of the list, which the wave's appends and the descriptor kernels' reads both
 // pay for: 130 M triplets took 140 of k_build's 506 us to store in 32 bits.
-template <bool NARROW>
+// W waves: each takes a contiguous part of the runs, counts its pairs, and
+// appends them behind those of the waves before it (the same list).
+template <bool NARROW, int W>
 __device__ __forceinline__ void triplets_from_lds(int i, int K, float4 *s_p, double rcA, const TripletBufs &tb,
-                                                  int lane) {
+                                                  int wv, int lane) {
   constexpr int kOwn = 4;  // register-held record chunks: K <= 64 kOwn
   constexpr int SH = NARROW ? 8 : 16;
   typedef typename std::conditional<NARROW, uint16_t, uint32_t>::type Entry;
@@ -362,14 +374,34 @@ __device__ __forceinline__ void triplets_from_lds(int i, int K, float4 *s_p, dou
   Entry *out = (Entry *)tb.list + (size_t)i * tb.tcap;
   int count = 0;
   // pairs of the step whose lanes pass `ok`, appended after `count` entries
-  auto emit = [&](bool ok, uint32_t pair) {
+  auto emit = [&](bool ok, uint32_t pair, auto store) {
     const unsigned long long m = __ballot(ok);
+    if (!decltype(store)::value) {
+      count += __popcll(m);
+      return;
+    }
     const unsigned pre = __builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
     if (ok && (int)pre < tb.tcap - count) out[count + pre] = (Entry)pair;
     count += __popcll(m);
   };
+  // this wave's steps d1 = first .. last of 1 .. K / 2
+  const int share = (K / 2 + W - 1) / W;
+  const int first = 1 + wv * share, last = min(K / 2, first + share - 1);
+  auto walk = [&](auto pass) {
+    if constexpr (W == 1) {
+      pass(std::true_type{});
+    } else {
+      __shared__ int s_pairs[W];
+      pass(std::false_type{});
+      if (lane == 0) s_pairs[wv] = count;
+      __syncthreads();
+      count = 0;
+      for (int w = 0; w < wv; ++w) count += s_pairs[w];
+      pass(std::true_type{});
+    }
+  };
   if (K <= 64 * kOwn) {
-    for (int t = lane; t < K / 2; t += 64) s_p[K + t] = s_p[t];
+    for (int t = 64 * wv + lane; t < K / 2; t += 64 * W) s_p[K + t] = s_p[t];
     __syncthreads();
     const int KX = K + K / 2;  // records readable at c + d
     // Q chunks of 64 neighbours: the records of U steps are read together, so
@@ -387,7 +419,7 @@ __device__ __forceinline__ void triplets_from_lds(int i, int K, float4 *s_p, dou
       }
       // one step: run d1 (K - d1 pairs) and run K - d1 (d1 pairs), or, when the
       // two are the same run (2 d1 = K), its n = K - d1 pairs only
-      auto batch = [&](int d0, int live) {
+      auto batch = [&](int d0, int live, auto store) {
         float4 pp[U][Q];
 #pragma unroll
         for (int u = 0; u < U; ++u)
@@ -404,12 +436,13 @@ __device__ __forceinline__ void triplets_from_lds(int i, int K, float4 *s_p, dou
             const float ex = pp[u][q].x - own[q].x, ey = pp[u][q].y - own[q].y, ez = pp[u][q].z - own[q].z;
             const bool ok = (ex * ex + ey * ey + ez * ez <= rc2) & (c < n);
             // run d1: (c, c + d1); run K - d1: (c + d1 - K, c)
-            emit(ok, self[q] + (c < n1 ? hi : lo));
+            emit(ok, self[q] + (c < n1 ? hi : lo), store);
           }
         }
       };
-      const int last = K / 2;  // steps d1 = 1 .. K / 2
-      for (int d0 = 1; d0 <= last; d0 += U) batch(d0, min(U, last - d0 + 1));
+      walk([&](auto store) {
+        for (int d0 = first; d0 <= last; d0 += U) batch(d0, min(U, last - d0 + 1), store);
+      });
     };
     typedef std::integral_constant<int, 1> C1;
     typedef std::integral_constant<int, 2> C2;
@@ -421,24 +454,26 @@ __device__ __forceinline__ void triplets_from_lds(int i, int K, float4 *s_p, dou
     else
       runs(C4{}, C1{});
   } else {
-    for (int d1 = 1; 2 * d1 <= K; ++d1) {
-      // run d1 (K - d1 pairs), then run d2 = K - d1 (d1 pairs) unless it is d1
-      const int d2 = K - d1;
-      const int n1 = K - d1, n = (d2 != d1) ? K : n1;
-      for (int c0 = 0; c0 < n; c0 += 64) {
-        const int c = c0 + lane;
-        const bool first = c < n1;
-        const int a = first ? c : c - n1, b = a + (first ? d1 : d2);
-        // both records read unconditionally (idle lanes read record 0) and
-        // the tests combined without short-circuits: one LDS round trip
-        const bool live = c < n;
-        const float4 pa = s_p[live ? a : 0], pb = s_p[live ? b : 0];
-        const float ex = pb.x - pa.x, ey = pb.y - pa.y, ez = pb.z - pa.z;
-        emit(live & (ex * ex + ey * ey + ez * ez <= rc2), (uint32_t)a | ((uint32_t)b << SH));
+    walk([&](auto store) {
+      for (int d1 = first; d1 <= last; ++d1) {
+        // run d1 (K - d1 pairs), then run d2 = K - d1 (d1 pairs) unless it is d1
+        const int d2 = K - d1;
+        const int n1 = K - d1, n = (d2 != d1) ? K : n1;
+        for (int c0 = 0; c0 < n; c0 += 64) {
+          const int c = c0 + lane;
+          const bool fore = c < n1;
+          const int a = fore ? c : c - n1, b = a + (fore ? d1 : d2);
+          // both records read unconditionally (idle lanes read record 0) and
+          // the tests combined without short-circuits: one LDS round trip
+          const bool live = c < n;
+          const float4 pa = s_p[live ? a : 0], pb = s_p[live ? b : 0];
+          const float ex = pb.x - pa.x, ey = pb.y - pa.y, ez = pb.z - pa.z;
+          emit(live & (ex * ex + ey * ey + ez * ez <= rc2), (uint32_t)a | ((uint32_t)b << SH), store);
+        }
       }
-    }
+    });
   }
-  if (lane == 0) {
+  if (lane == 0 && wv == W - 1) {
     tb.count[i] = min(count, tb.tcap);
     tb.raw[i] = count;
   }
@@ -452,17 +487,11 @@ struct ImageRec {
   double sx, sy, sz;
 };
 
-// Inclusive prefix sum over the wave by row shifts and row broadcasts.
-__device__ __forceinline__ int wave_prefix(int v) {
-#define GAPX_SCAN(ctrl, rows) v += __builtin_amdgcn_update_dpp(0, v, ctrl, rows, 0xf, false)
-  GAPX_SCAN(0x111, 0xf);  // row_shr:1
-  GAPX_SCAN(0x112, 0xf);  // row_shr:2
-  GAPX_SCAN(0x114, 0xf);  // row_shr:4
-  GAPX_SCAN(0x118, 0xf);  // row_shr:8
-  GAPX_SCAN(0x142, 0xa);  // row_bcast:15 into rows 1 and 3
-  GAPX_SCAN(0x143, 0xc);  // row_bcast:31 into rows 2 and 3
-#undef GAPX_SCAN
-  return v;
+// Order of LDS accesses within the one wave of a workgroup: the hardware keeps
+// it, the compiler has to be told.
+__device__ __forceinline__ void wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
 // One wavefront per centre atom.  The (2S+1)^3 bin images are taken 64 at a
@@ -478,17 +507,14 @@ __device__ __forceinline__ int wave_prefix(int v) {
 // neighbours the triplets took 220 (140 of them stores), the candidates 214, the
 // set-up 70.  16-bit triplets, LDS reads a batch of runs ahead, image records in
 // LDS instead of shuffles (a binary search of six and five fetches per
-// candidate) and a prefix sum by row shifts: 506 -> 433 us.
+// candidate) and a prefix sum by row shifts: 506 -> 433 us; the next group's and
+// batch's loads ahead of the current tests: 420 us.
 template <bool TRIP>
-__global__ __launch_bounds__(64) void k_build(int N, const int *__restrict__ atom_struct,
-                                              const StructParams *__restrict__ sp, double rcut, NeighborBufs nb,
-                                              double rcA, TripletBufs tb) {
-  extern __shared__ __align__(16) unsigned char smem[];
-  float4 *s_p = (float4 *)smem;  // [trip_lds_records(kcap)] with TRIP
+__device__ __forceinline__ int neighbour_list(int i, int lane, const int *__restrict__ atom_struct,
+                                              const StructParams *__restrict__ sp, double rcut,
+                                              const NeighborBufs &nb, double rcA, float4 *s_p) {
   __shared__ ImageRec s_rec[64];
   __shared__ int s_flag[64];
-  const int i = blockIdx.x, lane = threadIdx.x;
-  if (i >= N) return;
   s_flag[lane] = 0;
   int mark = 0;
   const StructParams &P = sp[atom_struct[i]];
@@ -529,10 +555,10 @@ __global__ __launch_bounds__(64) void k_build(int N, const int *__restrict__ ato
   const float M0 = fmaxf(R00, 0.f) + fmaxf(R01, 0.f) + fmaxf(R02, 0.f), M1r = fmaxf(R11, 0.f) + fmaxf(R12, 0.f);
   const float m2r = fminf(R22, 0.f), M2r = fmaxf(R22, 0.f);
   const float rp = (float)rcut + 0.01f, rp2 = rp * rp;
-  int count = 0;
-  for (int g0 = 0; g0 < nimg; g0 += 64) {
+  // bin range and lattice translation of image g0 + lane (n = 0: none)
+  auto image = [&](int g0, int &lo, int &n, int &t0, int &t1, int &t2) {
     const int img = g0 + lane;
-    int lo = 0, n = 0, t0 = 0, t1 = 0, t2 = 0;
+    lo = n = t0 = t1 = t2 = 0;
     if (img < nimg) {
       const int q2 = floordiv_small(img, inv_m2), q1 = floordiv_small(q2, inv_m1);
       const int o2 = img - q2 * m2 - P.S[2], o1 = q2 - q1 * m1 - P.S[1], o0 = q1 - P.S[0];
@@ -550,6 +576,15 @@ __global__ __launch_bounds__(64) void k_build(int N, const int *__restrict__ ato
         n = nb.bin_start[bin + 1] - lo;
       }
     }
+  };
+  int count = 0;
+  // the next group's bin ranges and the next batch's candidates are loaded before
+  // the current ones are tested: a small batch has no other wave to wait beside
+  int lo, n, t0, t1, t2;
+  image(0, lo, n, t0, t1, t2);
+  for (int g0 = 0; g0 < nimg; g0 += 64) {
+    int lo_n, n_n, t0_n, t1_n, t2_n;
+    image(g0 + 64, lo_n, n_n, t0_n, t1_n, t2_n);
     const int incl = wave_prefix(n);
     const int total = __builtin_amdgcn_readlane(incl, 63);
     const int excl = incl - n;
@@ -567,33 +602,48 @@ __global__ __launch_bounds__(64) void k_build(int N, const int *__restrict__ ato
       rec.sz = t0 * P.L[2] + t1 * P.L[5] + t2 * P.L[8];
       s_rec[below] = rec;
     }
-    for (int c0 = 0; c0 < total; c0 += 64) {
+    // candidate c0 + lane: its image's record and its atom's
+    auto candidate = [&](int c0, ImageRec &rec, int4 &inf, double2 &pxy, double &pz) {
       const int c = c0 + lane;
       // a lane's bin: the bins before this batch plus those that start at or
       // before the lane, which mark their first candidate's place
       ++mark;
       const int at = excl - c0;
       if (n > 0 && at >= 0 && at < 64) s_flag[at] = mark;
-      __syncthreads();
+      wave_order();
       const unsigned long long starts = __ballot(s_flag[lane] == mark);
       const int before = __popcll(__ballot(n > 0 && at < 0));
       const unsigned upto = __builtin_amdgcn_mbcnt_hi((unsigned)(starts >> 32),
                                                       __builtin_amdgcn_mbcnt_lo((unsigned)starts, 0u)) +
                             (unsigned)((starts >> lane) & 1ull);
-      const ImageRec rec = s_rec[max(before + (int)upto - 1, 0)];
-      __syncthreads();  // read before the next batch's marks
-      const int q = rec.first + c;
+      rec = s_rec[max(before + (int)upto - 1, 0)];
+      wave_order();  // read before the next batch's marks
+      const size_t q = (size_t)max(rec.first + min(c, total - 1), 0);
+      inf = sinfo[q];
+      pxy = sp2[2 * q];
+      pz = sp2[2 * q + 1].x;
+    };
+    ImageRec rec;
+    int4 inf;
+    double2 pxy;
+    double pz;
+    wave_order();
+    if (total > 0) candidate(0, rec, inf, pxy, pz);
+    for (int c0 = 0; c0 < total; c0 += 64) {
+      const int c = c0 + lane;
+      ImageRec rec_n = rec;
+      int4 inf_n = inf;
+      double2 pxy_n = pxy;
+      double pz_n = pz;
+      if (c0 + 64 < total) candidate(c0 + 64, rec_n, inf_n, pxy_n, pz_n);
       const int T0 = (rec.t & 255) - 64, T1 = ((rec.t >> 8) & 255) - 64, T2 = (rec.t >> 16) - 64;
       bool ok = false;
-      int4 inf = make_int4(0, 0, 0, 0);
       double dx = 0, dy = 0, dz = 0, r = 0;
       if (c < total) {
-        inf = sinfo[q];
-        const double2 pxy = sp2[2 * (size_t)q], pz = sp2[2 * (size_t)q + 1];
         if (!(T0 == 0 && T1 == 0 && T2 == 0 && inf.x == i)) {
           dx = pxy.x + rec.sx - xi;
           dy = pxy.y + rec.sy - yi;
-          dz = pz.x + rec.sz - zi;
+          dz = pz + rec.sz - zi;
           r = sqrt(dx * dx + dy * dy + dz * dz);
           ok = !(r > rcut);
         }
@@ -614,18 +664,54 @@ __global__ __launch_bounds__(64) void k_build(int N, const int *__restrict__ ato
         if (TRIP) s_p[pos] = trip_record(dx, dy, dz, r, trip_rc(rcA));
       }
       count += __popcll(m);
+      rec = rec_n;
+      inf = inf_n;
+      pxy = pxy_n;
+      pz = pz_n;
     }
+    lo = lo_n;
+    n = n_n;
+    t0 = t0_n;
+    t1 = t1_n;
+    t2 = t2_n;
   }
   if (lane == 0) {
     nb.nb_count[i] = min(count, nb.kcap);
     nb.nb_raw[i] = count;
   }
-  if (TRIP) {
+  return min(count, nb.kcap);
+}
+
+// W waves per atom: the first one builds the list, all of them its triplets.
+template <bool TRIP, int W>
+__global__ __launch_bounds__(64 * W) void k_build(int N, const int *__restrict__ atom_struct,
+                                                  const StructParams *__restrict__ sp, double rcut, NeighborBufs nb,
+                                                  double rcA, TripletBufs tb) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  float4 *s_p = (float4 *)smem;  // [trip_lds_records(kcap)] with TRIP
+  const int i = blockIdx.x, lane = threadIdx.x & 63;
+  if (i >= N) return;
+  if constexpr (W == 1) {
+    const int K = neighbour_list<TRIP>(i, lane, atom_struct, sp, rcut, nb, rcA, s_p);
+    if (TRIP) {
+      __syncthreads();
+      if (tb.narrow)
+        triplets_from_lds<true, 1>(i, K, s_p, rcA, tb, 0, lane);
+      else
+        triplets_from_lds<false, 1>(i, K, s_p, rcA, tb, 0, lane);
+    }
+  } else {
+    __shared__ int s_K;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (wv == 0) {
+      const int K = neighbour_list<TRIP>(i, lane, atom_struct, sp, rcut, nb, rcA, s_p);
+      if (lane == 0) s_K = K;
+    }
     __syncthreads();
     if (tb.narrow)
-      triplets_from_lds<true>(i, min(count, nb.kcap), s_p, rcA, tb, lane);
+      triplets_from_lds<true, W>(i, s_K, s_p, rcA, tb, wv, lane);
     else
-      triplets_from_lds<false>(i, min(count, nb.kcap), s_p, rcA, tb, lane);
+      triplets_from_lds<false, W>(i, s_K, s_p, rcA, tb, wv, lane);
   }
 }
 
@@ -644,7 +730,7 @@ __global__ __launch_bounds__(64) void k_triplets_from_slots(int N, NeighborBufs 
     s_p[a] = trip_record(d[0], d[1], d[2], d[3], trip_rc(rcA));
   }
   __syncthreads();
-  triplets_from_lds<false>(i, K, s_p, rcA, tb, lane);
+  triplets_from_lds<false, 1>(i, K, s_p, rcA, tb, 0, lane);
 }
 
 // |pos_i - (pos_j + n1 L1 + n2 L2 + n3 L3)| in the order of operations of
@@ -1061,13 +1147,33 @@ hipError_t launch_bin_structures(hipStream_t s, int nstruct, const double *pos, 
   return hipGetLastError();
 }
 
+// Waves per atom of k_build.  The triplets are a serial chain of about 250 cycles
+// per 64 pairs for one wave (10 of the kernel's 18 us at 77 neighbours), so while
+// the chip has wave slots to spare several waves share them.  One, four and eight
+// waves, us a replayed evaluation: 8 atoms 70.4 65.1 63.7, 256 76.3 71.6 70.2, 768
+// 95.2 90.1 89.3, 1024 104.5 97.2 103.6, 1536 126.6 123.4 130.6, 2048 132.3 137.9
+// 143.6.
+static int build_waves(int N) { return N <= 768 ? 8 : N <= 1536 ? 4 : 1; }
+
+template <int W>
+static hipError_t launch_build(hipStream_t s, int N, const int *atom_struct, const StructParams *sp, double rcut,
+                               const NeighborBufs &nb, double rcA, const TripletBufs &tb) {
+  const size_t lds = sizeof(float4) * trip_lds_records(nb.kcap);
+  k_build<true, W><<<N, 64 * W, lds, s>>>(N, atom_struct, sp, rcut, nb, rcA, tb);
+  return hipGetLastError();
+}
+
 hipError_t launch_build_neighbors(hipStream_t s, int N, const int *atom_struct, const StructParams *sp,
                                   double rcut, NeighborBufs nb, double rcA, const TripletBufs *tb) {
-  if (tb)
-    k_build<true><<<N, 64, sizeof(float4) * trip_lds_records(nb.kcap), s>>>(N, atom_struct, sp, rcut, nb, rcA, *tb);
-  else
-    k_build<false><<<N, 64, 0, s>>>(N, atom_struct, sp, rcut, nb, 0.0, TripletBufs{});
-  return hipGetLastError();
+  if (!tb) {
+    k_build<false, 1><<<N, 64, 0, s>>>(N, atom_struct, sp, rcut, nb, 0.0, TripletBufs{});
+    return hipGetLastError();
+  }
+  switch (build_waves(N)) {
+    case 8: return launch_build<8>(s, N, atom_struct, sp, rcut, nb, rcA, *tb);
+    case 4: return launch_build<4>(s, N, atom_struct, sp, rcut, nb, rcA, *tb);
+    default: return launch_build<1>(s, N, atom_struct, sp, rcut, nb, rcA, *tb);
+  }
 }
 
 hipError_t launch_triplets_from_slots(hipStream_t s, int N, NeighborBufs nb, double rcA, TripletBufs tb) {
