@@ -671,13 +671,16 @@ static double best_splits(int tiles, int slots, int chunks, double over, double 
 // The contraction's split used to aim at 512 workgroups whatever the tiles:
 // 67,647 atoms gave 1058 FP64 workgroups for the chip's 512 places and 529
 // mixed ones (a second round for 17 of them).  Measured there, us by splits:
-// FP64 1: 2700, 3: 2440, 4: 2365, 6: 2303; mixed 1: 489, 2: 403, 3: 381,
-// 4: 373, 6: 364, 8: 380, the backward then 3 (mixed) or 6 us (FP64) longer
+// FP64 1: 2700, 3: 2440, 4: 2365, 6: 2303; mixed 1: 492, 2: 406, 3: 384,
+// 4: 372, 6: 364, 8: 380, the backward then 3 (mixed) or 6 us (FP64) longer
 // per split.  At 4096 atoms the rule keeps one full round (FP64 8 splits
 // 157 us, 12: 176, 16: 167; mixed 36 for 64- and 128-row tiles); at 197 atoms
-// 64-row tiles give twice the workgroups (11.3 against 13.9 us).  A chunk of
-// 64 points takes a workgroup about 16 us in FP64 and 3.9 us mixed (128 rows,
-// D = 128; 64 rows 0.71 of it), its start and end 0.2 FP64 and three mixed ones.
+// 64-row tiles give twice the workgroups (11.0 against 13.7 us), and a split's
+// partials cost the backward a tenth of a microsecond however few the atoms (its
+// reads are one round trip per eight: 32 splits 11.6 + 18.4 us, 63: 11.0 + 21.6).
+// A chunk of 64 points takes a workgroup about 16 us in FP64 and 3.9 us mixed
+// (128 rows, D = 128; 64 rows 0.71 of it), its start and end 0.2 FP64 and three
+// mixed ones.
 static void default_tuning(Ctx &c) {
   const Model &m = *c.m;
   for (int p = 0; p < 2; ++p) {
@@ -685,15 +688,15 @@ static void default_tuning(Ctx &c) {
     Tuning &t = c.tune[p];
     const bool fp64 = p == 0, c64 = fp64 || m.mixed_f64, grid = m.sfd.grid != 0;
     // two overlapped halves pay only where the contraction leaves registers
-    // free (replayed 67,647 atoms: mixed 1729 against 1754 us, FP64 5055
-    // against 5100 but eager 5190 against 5100; 32,768 atoms with D = 256,
-    // one workgroup a CU, 2341 against 2323, eager 2460 against 2300)
+    // free (replayed 67,647 atoms: mixed 1654 against 1687 us, FP64 4871
+    // against 4926 but eager 5026 against 4938; 32,768 atoms with D = 256,
+    // one workgroup a CU, 2186 against 2164, eager 2326 against 2150)
     t.halves = (!c64 && m.Dp <= 128) ? 1 : 0;
     if (!c.waves_fwd_given) t.waves_fwd = waves_within(c.N, fwd_wave_cap(fp64), 1);
     if (!c.waves_bwd_given) t.waves_bwd = waves_within(c.N, bwd_wave_cap(fp64, grid), !grid ? 4 : 1);
     const int pts = gpr_points_per_chunk(m.Dp), chunks = m.Mp / pts;
     const double scale = m.Dp / 128.0 * pts / 64.0;
-    const double part_us = (double)c.Np * m.Dp * (c64 ? 8 : 4) / 1e7;
+    const double part_us = std::max(0.1, (double)c.Np * m.Dp * (c64 ? 8 : 4) / 1e7);
     if (c64) {
       const int tiles = c.Np / 64, slots = m.Dp <= 160 ? 512 : 256;
       int s = 1;
