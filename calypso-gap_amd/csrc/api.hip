@@ -434,7 +434,7 @@ static const char *kStageNames[kNumStages] = {"neighbor_list", "descriptors_fwd"
 // Launch shapes chosen per context and precision (defaults, environment
 // overrides, or gapx_ctx_autotune).
 struct Tuning {
-  int waves_fwd = 4, waves_bwd = 4;  // wavefronts per atom in the descriptor kernels
+  int waves_fwd = 4, waves_bwd = 4;  // wavefronts per atom in the descriptor kernels (1, 2, 4, 8)
   int gpr_rows = 64;                 // rows per workgroup of the contraction (64 or 128)
   int gpr_blocks = 512;              // target workgroups of the contraction (sets the splits)
   int halves = 1;                    // the two-half schedule where the batch allows it (1) or one piece (0)
@@ -692,8 +692,8 @@ static void default_tuning(Ctx &c) {
     // against 4926 but eager 5026 against 4938; 32,768 atoms with D = 256,
     // one workgroup a CU, 2186 against 2164, eager 2326 against 2150)
     t.halves = (!c64 && m.Dp <= 128) ? 1 : 0;
-    if (!c.waves_fwd_given) t.waves_fwd = waves_within(c.N, fwd_wave_cap(fp64), 1);
-    if (!c.waves_bwd_given) t.waves_bwd = waves_within(c.N, bwd_wave_cap(fp64, grid), !grid ? 4 : 1);
+    if (!c.waves_fwd_given) t.waves_fwd = default_waves_fwd(c.N, fp64);
+    if (!c.waves_bwd_given) t.waves_bwd = default_waves_bwd(c.N, fp64, grid);
     const int pts = gpr_points_per_chunk(m.Dp), chunks = m.Mp / pts;
     const double scale = m.Dp / 128.0 * pts / 64.0;
     const double part_us = std::max(0.1, (double)c.Np * m.Dp * (c64 ? 8 : 4) / 1e7);
@@ -1483,8 +1483,8 @@ static int ctx_autotune(Ctx &c, int flags, bool force) {
     std::vector<int> values;
   };
   std::vector<Knob> knobs;
-  knobs.push_back({&t.waves_fwd, {1, 2, 4}});
-  if (flags & GAPX_GRAD) knobs.push_back({&t.waves_bwd, {1, 2, 4}});
+  knobs.push_back({&t.waves_fwd, {1, 2, 4, 8}});
+  if (flags & GAPX_GRAD) knobs.push_back({&t.waves_bwd, {1, 2, 4, 8}});
   // the descriptor kernels' waves one knob at a time
   auto descend = [&]() {
     for (Knob &k : knobs) {
@@ -2864,8 +2864,9 @@ int gapx_ctx_get_tuning(gapx_ctx *c, int flags, int *waves_fwd, int *waves_bwd, 
                         int *halves) {
   if (!c) return fail(GAPX_ERR_ARG, "null context");
   const Tuning &t = c->tune[(run_flags(*c->m, flags) & GAPX_MIXED) ? 1 : 0];
-  if (waves_fwd) *waves_fwd = t.waves_fwd;
-  if (waves_bwd) *waves_bwd = t.waves_bwd;
+  // within set_tuning's range: eight, which only a load or the autotuner picks, as four
+  if (waves_fwd) *waves_fwd = std::min(t.waves_fwd, 4);
+  if (waves_bwd) *waves_bwd = std::min(t.waves_bwd, 4);
   if (gpr_rows) *gpr_rows = t.gpr_rows;
   if (gpr_blocks) *gpr_blocks = t.gpr_blocks;
   if (halves) *halves = t.halves;

@@ -1771,7 +1771,6 @@ hipError_t launch_descriptors_fwd(hipStream_t s, bool fp64, int N, const int *sp
                                   int waves, int KP, int atom0) {
   Lds L{KP, sf.n_groups > 0 ? sf.n_groups : 1, out.Dp, atom0, sf.n_rad};
   if (N <= 0) return hipSuccess;
-  waves = widened(waves, N, fwd_wave_cap(fp64));
   if (sf.grid) {
     if (fp64) return fwd_grid<double>(waves, s, N, species, wz, nb, tb, sf, L, theta_inv, mu, split_mode, out);
     return fwd_grid<float>(waves, s, N, species, wz, nb, tb, sf, L, theta_inv, mu, split_mode, out);
@@ -1792,7 +1791,6 @@ hipError_t launch_descriptors_bwd(hipStream_t s, bool fp64, int N, const int *sp
   if (N <= 0) return hipSuccess;
   // the LDS layout's 16-byte reads of g need KP (slots per atom) a multiple of 4
   if (KP % 4 != 0) return hipErrorInvalidValue;
-  waves = widened(waves, N, bwd_wave_cap(fp64, sf.grid != 0));
   if (fp64) return bwd_fit<double>(waves, s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
   return bwd_fit<float>(waves, s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
 }

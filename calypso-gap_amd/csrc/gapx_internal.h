@@ -322,13 +322,17 @@ hipError_t launch_descriptors_bwd(hipStream_t s, bool fp64, int N, const int *sp
 //   generic FP64   64: 168 98 78 63 forward, 237 131 76 48 backward;
 //                  1024: 205 139 169 233, 273 173 158 178;  4096: 397 497 635 914, 793 541 462 685
 // so W is the largest with N W within these waves; the generic backward keeps
-// four whatever N.
+// at least four whatever N.
 constexpr int fwd_wave_cap(bool fp64) { return fp64 ? 3072 : 4096; }
 constexpr int bwd_wave_cap(bool fp64, bool grid) { return !grid ? 5120 : fp64 ? 2560 : 4096; }
-// The launchers run four waves per atom as eight where N allows it.
-constexpr int widened(int waves, int N, int cap) { return waves == 4 && (long long)N * 8 <= cap ? 8 : waves; }
 constexpr int waves_within(int N, int cap, int least) {
-  return (long long)N * 4 <= cap ? 4 : (long long)N * 2 <= cap ? 2 > least ? 2 : least : least;
+  for (int w = 8; w > least; w /= 2)
+    if ((long long)N * w <= cap) return w;
+  return least;
+}
+constexpr int default_waves_fwd(int N, bool fp64) { return waves_within(N, fwd_wave_cap(fp64), 1); }
+constexpr int default_waves_bwd(int N, bool fp64, bool grid) {
+  return waves_within(N, bwd_wave_cap(fp64, grid), grid ? 1 : 4);
 }
 
 // Largest per-atom neighbour count the descriptor kernels take: within the

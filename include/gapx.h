@@ -274,6 +274,12 @@ int gapx_ctx_momenta(gapx_ctx *c, double *p);
  * results are cached per process for the shape class unless force != 0.
  * No reference counterpart. */
 int gapx_ctx_autotune(gapx_ctx *c, int flags, int force);
+/* The launch shapes themselves.  Until they are given here or autotuned, every
+ * load picks them by the batch's size; given ones stay across loads and run as
+ * given.  waves_fwd, waves_bwd: 1, 2 or 4 wavefronts per atom (the forward of
+ * grid-form tables has no form with four and runs two; long neighbour lists
+ * fall back to fewer); small batches are given eight by a load or the
+ * autotuner, which get_tuning reports as 4. */
 int gapx_ctx_get_tuning(gapx_ctx *c, int flags, int *waves_fwd, int *waves_bwd, int *gpr_rows, int *gpr_blocks,
                         int *halves);
 int gapx_ctx_set_tuning(gapx_ctx *c, int flags, int waves_fwd, int waves_bwd, int gpr_rows, int gpr_blocks,
