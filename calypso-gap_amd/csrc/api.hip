@@ -1235,6 +1235,16 @@ static int enqueue_run(Ctx &c, int flags) {
   return enqueue_forces(c, b, fp64, grad, g.eatom, gs, tu.waves_bwd);
 }
 
+// Waves per atom of the surrogate's forward, one (grid tables) or four (others)
+// for every batch unless the caller gave a shape: more waves add FP32 features in
+// another order, and the surrogate rounds them to BF16, where a last bit can
+// become a whole step, so that a structure's energy would depend on how many
+// share its call (energies of 24 atoms alone and among 60 copies differed).
+static int surrogate_waves_fwd(const Ctx &c, int p) {
+  if (c.tune_given[p] || c.waves_fwd_given) return c.tune[p].waves_fwd;
+  return c.m->sfd.grid ? 1 : 4;
+}
+
 // The surrogate in place of the contraction: same neighbour lists and
 // descriptors, MLP energies and dE/dx, same backward pass.  The MLP time is
 // reported as the contraction stage.
@@ -1263,7 +1273,8 @@ static int enqueue_surrogate(Ctx &c, Mlp &mlp, int flags) {
   const Tuning &tu = c.tune[fp64 ? 0 : 1];
   stage_begin(c, kDescFwd);
   GAPX_HIP(launch_descriptors_fwd(c.stream, fp64, c.N, c.d_species, m.d_wz, b.nb, b.tb, m.sfd,
-                                  m.d_theta_inv, m.d_mu, 0, o, c.chunk > 0 ? c.chunk : 16, tu.waves_fwd, c.KP));
+                                  m.d_theta_inv, m.d_mu, 0, o, c.chunk > 0 ? c.chunk : 16,
+                                  surrogate_waves_fwd(c, fp64 ? 0 : 1), c.KP));
   stage_end(c, kDescFwd);
   if (grad && (rc = fork_reverse(c, b))) return rc;
   float *xin = o.xt32;
