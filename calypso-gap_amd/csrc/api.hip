@@ -2002,8 +2002,12 @@ static int ctx_car2acsf(Ctx &c, int na, int max_nb, int nf, const double *pos, c
     GAPX_HIP(launch_fill_int(c.stream, tb.count, N, 0));
   o.N = N;
   o.Dp = Dp;
+  // shapes by this table's size, as a load picks them by its batch's; those in
+  // c.tune are the context's last evaluation's
+  const int waves_fwd = c.waves_fwd_given ? c.tune[0].waves_fwd : default_waves_fwd(N, true);
+  const int waves_bwd = c.waves_bwd_given ? c.tune[0].waves_bwd : default_waves_bwd(N, true, m.sfd.grid != 0);
   GAPX_HIP(launch_descriptors_fwd(c.stream, true, N, nullptr, m.d_wz, nb, tb, m.sfd, m.d_theta_inv, m.d_mu, 0, o,
-                                  c.chunk > 0 ? c.chunk : 16, c.tune[0].waves_fwd, kcap));
+                                  c.chunk > 0 ? c.chunk : 16, waves_fwd, kcap));
   std::vector<double> hx((size_t)N * Dp);
   GAPX_HIP(hipMemcpyAsync(hx.data(), o.x64, sizeof(double) * hx.size(), hipMemcpyDeviceToHost, c.stream));
   GAPX_HIP(hipStreamSynchronize(c.stream));
@@ -2026,7 +2030,7 @@ static int ctx_car2acsf(Ctx &c, int na, int max_nb, int nf, const double *pos, c
       }
       GAPX_HIP(hipMemcpyAsync(g64, hg.data(), sizeof(double) * hg.size(), hipMemcpyHostToDevice, c.stream));
       GAPX_HIP(launch_descriptors_bwd(c.stream, true, N, nullptr, m.d_wz, nb, tb, m.sfd, Dp, gs, slot_f, vir,
-                                      c.tune[0].waves_bwd, kcap));
+                                      waves_bwd, kcap));
       GAPX_HIP(hipMemcpyAsync(hs.data(), slot_f, sizeof(double) * hs.size(), hipMemcpyDeviceToHost, c.stream));
       GAPX_HIP(hipMemcpyAsync(hv.data(), vir, sizeof(double) * hv.size(), hipMemcpyDeviceToHost, c.stream));
       GAPX_HIP(hipStreamSynchronize(c.stream));
