@@ -301,20 +301,22 @@ static int upload_model(Model &m) {
 #define PUT(dst, vec, T)                                                                     \
   GAPX_HIP(put(dst, (vec).empty() ? (const void *)zero.data() : (const void *)(vec).data(), \
                std::max<size_t>(1, (vec).size()) * sizeof(T)))
-  // Exponential coefficients beyond 1e20 / A^2 are cut there (such a term is 0
-  // at every distance above 1e-9 A either way), so that the kernels' exponents
-  // stay finite.
-  auto finite = [](std::vector<double> v) {
-    for (double &x : v) x = std::min(std::max(x, -1e20), 1e20);
+  // Exponential coefficients beyond +-1e20 / A^2 and centres beyond +-1e9 A are
+  // cut there, so that the kernels' exponents stay within 1e38 (exp64).  Cut or
+  // not, a term is 0 (coefficient above 0) or infinite (below) wherever the
+  // distance to its centre is above 3e-9 A.
+  auto within = [](std::vector<double> v, double lim) {
+    for (double &x : v) x = std::min(std::max(x, -lim), lim);
     return v;
   };
-  const std::vector<double> rad_av = finite(t.rad_a), ang_etav = finite(t.ang_eta);
+  const std::vector<double> rad_av = within(t.rad_a, 1e20), ang_etav = within(t.ang_eta, 1e20),
+                            rad_rsv = within(t.rad_rs, 1e9);
   std::vector<double> pirc;
   for (double rc : t.group_rc) pirc.push_back(kPi / rc);
-  PUT(rad_a, rad_av, double); PUT(rad_rs, t.rad_rs, double);
+  PUT(rad_a, rad_av, double); PUT(rad_rs, rad_rsv, double);
   {
     // the same tables rounded to FP32 for the FP32 kernels (no conversion per line)
-    std::vector<float> a32(rad_av.begin(), rad_av.end()), rs32(t.rad_rs.begin(), t.rad_rs.end());
+    std::vector<float> a32(rad_av.begin(), rad_av.end()), rs32(rad_rsv.begin(), rad_rsv.end());
     std::vector<float> fzero(1, 0.f);
     GAPX_HIP(put(rad_a32, a32.empty() ? fzero.data() : a32.data(), std::max<size_t>(1, a32.size()) * 4));
     GAPX_HIP(put(rad_rs32, rs32.empty() ? fzero.data() : rs32.data(), std::max<size_t>(1, rs32.size()) * 4));
@@ -1954,8 +1956,12 @@ static int ctx_car2acsf(Ctx &c, int na, int max_nb, int nf, const double *pos, c
   for (int i = 0; i < N; ++i)
     for (int a = 0; a < count[i]; ++a) {
       const size_t sl = (size_t)i * kcap + a;
-      for (int x = 0; x < 3; ++x) hd[4 * sl + x] = tab(i, a, x) - pos[i + (size_t)na * x];
-      hd[4 * sl + 3] = tab(i, a, 3);
+      // entries beyond 1e9 A, where every cutoff function is 0, are taken there
+      // with a zero vector: the kernels' exponents stay finite (those of an
+      // entry at 1e30 A gave NaN, and NaN times 0 is not 0)
+      const bool far = tab(i, a, 3) > 1e9;
+      for (int x = 0; x < 3; ++x) hd[4 * sl + x] = far ? 0.0 : tab(i, a, x) - pos[i + (size_t)na * x];
+      hd[4 * sl + 3] = far ? 1e9 : tab(i, a, 3);
       hw[sl] = tab(i, a, 4);
       const double jd = tab(i, a, 5);
       if (!(jd >= 1.0 && jd < na + 1.0)) return fail(GAPX_ERR_ARG, "gapx_car2acsf: neighbour index outside [1, NA]");

@@ -59,7 +59,9 @@ __device__ __forceinline__ double sconst(double c) {
 
 // exp(y): y = n ln2 + r, |r| <= ln2 / 2, 1 + r + r^2 q(r) with q of degree 9
 // (fit error 3.4e-18), scaled by 2^n.  Underflows to 0 and overflows to
-// infinity through the scaling; y must be finite.
+// infinity through the scaling.  y must be within about 1e40: past 2^53 the
+// remainder r grows with y's spacing, and its powers would overflow.  (The host
+// keeps coefficients within 1e20, centres and a caller's distances within 1e9 A.)
 __device__ __forceinline__ double exp64(double y) {
   const double n = __builtin_rint(y * sconst(1.4426950408889634));
   double r = fma(n, sconst(-6.93147180559945286e-01), y);

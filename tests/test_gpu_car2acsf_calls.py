@@ -1,9 +1,11 @@
 """CAR2ACSF from a caller's neighbour table: independent of the evaluations the
-model made before."""
+model made before, and of table entries far beyond every cutoff.  Lines centred
+far beyond their cutoff likewise, in every call."""
 import numpy as np
 import pytest
 
 import gapx
+import oracle
 from gapx import synth
 from test_gpu_descriptor_forms import FORMS, model_for
 
@@ -52,3 +54,46 @@ def test_same_bits_after_any_evaluation(form):
         print(form, copies, flush=True)
         for a, b in zip(out, ref):
             assert np.array_equal(a, b), copies
+
+
+# entries beyond every cutoff count nothing (a line's term needs r <= rc); the
+# sums in another order: 1e-12 of the largest value
+@pytest.mark.parametrize("far", [7.5, 1e9, 1e30, 1e200, np.inf])
+@pytest.mark.parametrize("form", ["eta3_zeta5", "eta4_two_radial_cutoffs", "no_grid"])
+def test_entries_beyond_the_cutoffs(form, far):
+    s, m = case(form)
+    nb, count = table(s, WEIGHT)
+    ref = m.car2acsf(s["pos"], nb, count)
+    for ahead in (False, True):  # behind each atom's row at a unit vector's place, before it at their own
+        wide = nb.copy()
+        for i, c in enumerate(count):
+            entry = np.r_[s["pos"][i] + [far if ahead else 1.0, 0, 0], far, 1.0, 1.0]
+            wide[i, :c + 1] = np.vstack([entry, nb[i, :c]] if ahead else [nb[i, :c], entry])
+        out = m.car2acsf(s["pos"], wide, count + 1)
+        print(form, far, ahead, flush=True)
+        for a, b in zip(out, ref):
+            assert np.isfinite(a).all()
+            assert np.abs(a - b).max() <= 1e-12 * max(1.0, np.abs(b).max())
+
+
+# a radial line centred there has no term; FP64 against the oracle at the parity
+# bar, mixed against FP64 (1e-5 of the sum of |E_i|, 1e-4 of the largest force)
+@pytest.mark.parametrize("rs", [1e9, 1e30, 1e200])
+@pytest.mark.parametrize("form", ["eta3_zeta5", "no_grid"])
+def test_lines_centred_beyond_their_cutoff(form, rs):
+    t, a, c, z = FORMS[form]
+    sf = (np.r_[t, 3].astype(np.int32), np.r_[a, rs], np.r_[c, 6.0], np.r_[z, 1.0])
+    s = synth.structure(9, 9 * 14.0, (1, 8, 22), np.random.default_rng(3), min_dist=1.3)
+    om = model_for(sf, s, np.random.default_rng(4))
+    ref = oracle.gap_calc(om, s["species"], s["lat"], s["pos"], 6.0, mode="sparse", nthreads=4)
+    m = gapx.Model.from_model(om)
+    ctx = gapx.Context(m)
+    ctx.load([s], 6.0)
+    ctx.run(gapx.GRAD)
+    r = ctx.results()
+    assert abs(r["energy"][0] - ref["energy"]) / 9 < 1e-9
+    assert np.abs(r["forces"] - ref["forces"]).max() < 1e-7
+    ctx.run(gapx.GRAD | gapx.MIXED)
+    x = ctx.results()
+    assert abs(x["energy"][0] - r["energy"][0]) < 1e-5 * np.abs(r["eatom"]).sum()
+    assert np.abs(x["forces"] - r["forces"]).max() < 1e-4 * np.abs(r["forces"]).max()
