@@ -75,6 +75,12 @@ def zeta_1_2_4_16(header):
     return sorted(set(np.round(header["sf_zeta"][ang]).astype(int).tolist())) == [1, 2, 4, 16]
 
 
+def angular_etas(header):
+    """Number of distinct etas of the angular lines."""
+    ang = np.isin(header["sf_type"], (2, 4))
+    return len(set(header["sf_alpha"][ang].tolist()))
+
+
 def contraction_grid(n_atoms, des_len, nsparse, mixed, tune):
     """Threads of one contraction launch over n_atoms rows (the host's split
     of the sparse points over grid.y for the tuned workgroup target)."""
@@ -89,11 +95,14 @@ def contraction_grid(n_atoms, des_len, nsparse, mixed, tune):
     return tiles * splits * (512 if (mixed and dp > 128) else 256)
 
 
-def stage_kernel(stage, mixed, tune, z16, des_len, n_atoms, nsparse, c64=False):
+def stage_kernel(stage, mixed, tune, z16, des_len, n_atoms, nsparse, c64=False, n_eta=4):
     """The one kernel of a single-kernel stage under the given launch shapes,
     as rocprofv3 names it, and its grid in threads for a one-piece launch over
     n_atoms (grid-form tables with 4 zetas; z16: the zeta list is {1, 2, 4,
-    16}; c64: the mixed run contracts in FP64).  The contraction is
+    16}; c64: the mixed run contracts in FP64; n_eta: etas of the table).  The
+    backward's third argument is its form: 4 zetas, plus 10 where it holds five
+    to eight etas in registers (FP32) or 20 where it reads them from LDS (more
+    than eight, FP64 more than four).  The contraction is
     instantiated for the descriptor length padded to 32; the mixed one as
     <bf16, D, row blocks per wave, waves>: four waves of one or two 16-row
     blocks up to 128 features, eight waves of one block above."""
@@ -104,7 +113,8 @@ def stage_kernel(stage, mixed, tune, z16, des_len, n_atoms, nsparse, c64=False):
         return "k_desc_fwd_grid<%s, 4, %d, %s, false>" % (t, w, z), n_atoms * 64 * w
     if stage == "descriptors_bwd":
         w = tune["waves_bwd"]
-        return "k_desc_bwd<%s, %d, 4, %s, false>" % (t, w, z), n_atoms * 64 * w
+        form = 4 if n_eta <= 4 else 14 if mixed and n_eta <= 8 else 24
+        return "k_desc_bwd<%s, %d, %d, %s, false>" % (t, w, form, z), n_atoms * 64 * w
     if stage == "gpr_contraction":
         dp = (des_len + 31) // 32 * 32
         grid = contraction_grid(n_atoms, des_len, nsparse, mixed and not c64, tune)
@@ -229,7 +239,8 @@ def measure(m, structs, rc, steps, warmup, label):
     rates = stage_rates(st, N, D, M, pairs, triplets, m, mixed=True)
     # the dominant kernel: the longest of the stages that are one kernel each
     dom = max(SINGLE_KERNEL_STAGES, key=lambda k: st[k])
-    kname, grid = stage_kernel(dom, True, runs["mixed"]["tune"], zeta_1_2_4_16(m.header()), D, N, M, c64)
+    kname, grid = stage_kernel(dom, True, runs["mixed"]["tune"], zeta_1_2_4_16(m.header()), D, N, M, c64,
+                               n_eta=angular_etas(m.header()))
     roof = {kk: rates[dom][kk] for kk in ("bound", "achieved", "peak", "unit", "frac")}
     roof["traffic"] = measured_traffic(label, kname, grid)
     roof["counters"] = measured_counters(label, kname, grid)
@@ -237,7 +248,8 @@ def measure(m, structs, rc, steps, warmup, label):
     roof["stages"] = {k: dict(ms=round(st[k], 4), **{kk: vv for kk, vv in rates[k].items()
                                                      if kk in ("achieved", "frac", "bound", "unit")}) for k in st}
     for k in SINGLE_KERNEL_STAGES:
-        kn, g = stage_kernel(k, True, runs["mixed"]["tune"], zeta_1_2_4_16(m.header()), D, N, M, c64)
+        kn, g = stage_kernel(k, True, runs["mixed"]["tune"], zeta_1_2_4_16(m.header()), D, N, M, c64,
+                               n_eta=angular_etas(m.header()))
         roof["stages"][k].update(kernel=kn, traffic=measured_traffic(label, kn, g),
                                  counters=measured_counters(label, kn, g))
     sec = runs["mixed"]["sec"]
