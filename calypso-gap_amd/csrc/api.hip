@@ -992,10 +992,10 @@ static int gpr_layout(Ctx &c, GprArgs &g, bool f64_kernel, int tune) {
   g.Dp = m.Dp;
   g.Mp = m.Mp;
   // the mixed kernel above D = 128 runs 128-row tiles only (eight waves
-  // sharing one workgroup's two chunk buffers)
+  // sharing one workgroup's four half-chunk buffers)
   g.rows = f64_kernel ? 64 : m.Dp > 128 ? 128 : t.gpr_rows == 128 ? 128 : 64;
   // Split the sparse points over grid.y until there are about gpr_blocks
-  // workgroups (resident waves; more splits only add partial-sum traffic).
+  // workgroups (default_tuning's or the caller's target).
   const int tiles = c.Np / g.rows;
   const int chunk = gpr_points_per_chunk(m.Dp);
   int splits = std::max(1, (t.gpr_blocks + tiles - 1) / tiles);

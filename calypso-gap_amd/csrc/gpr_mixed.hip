@@ -390,7 +390,8 @@ __global__ __launch_bounds__(64 * NW, 8 / NW) void k_gpr_mixed(GprArgs a) {
   gpr_mixed<BF, DP, R, NW, true>(a);
 }
 
-// Energies only: no feature-major halves, no second product.
+// Energies only: no feature-major loads, no second product (the halves' place in
+// LDS stays; only the chunk's norm terms and alphas are kept there).
 template <bool BF, int DP, int R, int NW>
 __global__ __launch_bounds__(64 * NW, 8 / NW) void k_gpr_mixed_energy(GprArgs a) {
   gpr_mixed<BF, DP, R, NW, false>(a);
@@ -406,7 +407,7 @@ void launch_one(hipStream_t s, const GprArgs &a, int tiles) {
 
 // rows per workgroup: 64 (four waves of one 16-row block) or 128 (four
 // waves of two blocks up to DP = 128; eight waves of one block above, where
-// two chunk buffers fill the LDS of a CU)
+// the four half-chunk buffers fill most of a CU's LDS)
 template <bool BF, int DP, bool GRAD>
 hipError_t launch_rows(hipStream_t s, const GprArgs &a) {
   const int tiles = a.ntiles > 0 ? a.ntiles : a.Np / a.rows;

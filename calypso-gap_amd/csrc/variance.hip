@@ -155,8 +155,9 @@ __global__ __launch_bounds__(256) void k_var_quad(int N, int r0, int Mp, const d
 // 16 accumulators, so a step of 4 points reads 8 operands from LDS for 16
 // products (5 for 4 above); the next 16 points travel to registers while the
 // current ones multiply, and go to the other LDS buffer behind them, with one
-// barrier per chunk: 48 -> 64 TF/s (2048 atoms, 4032 points, 1168 -> 1063 us; the
-// matrix cores 93 % busy at the 2.1 GHz the card runs here).  Rows of A are 18 doubles apart, rows of B 144: operand
+// barrier per chunk: 2048 atoms, 4032 points 1218 -> 1089 us (55 -> 61 TF/s), 4096
+// atoms 2351 -> 2149 (57 -> 62), kernel alone; the matrix cores 93 % busy at the
+// 2.1 GHz the card runs here.  Rows of A are 18 doubles apart, rows of B 144: operand
 // reads of 32 lanes fall on 64 different banks.  A tile's edge rows (rows is a multiple of 64) and columns repeat the
 // last one and are not stored; the partials are those of k_var_quad, in its
 // order of operations.
