@@ -81,6 +81,32 @@ __device__ __forceinline__ double exp64(double y) {
   return __builtin_amdgcn_ldexp(q, (int)n);
 }
 
+// The same with the constants held by the caller, for a loop that a single wave
+// runs on its SIMD: formed per call they are 23 scalar moves, which that wave
+// pays for in full.  (Elsewhere the moves hide behind other waves, and all of
+// them ahead of the polynomial cost 1 % of an FP64 evaluation.)
+struct ExpConst {
+  double log2e, ln2_hi, ln2_lo, q[10];
+  __device__ __forceinline__ ExpConst()
+      : log2e(sconst(1.4426950408889634)), ln2_hi(sconst(-6.93147180559945286e-01)),
+        ln2_lo(sconst(-2.31904681384629956e-17)),
+        q{sconst(2.5117915126746086e-08), sconst(2.76313397049011e-07), sconst(2.755721613139287e-06),
+          sconst(2.480148978582598e-05), sconst(0.00019841269917571867), sconst(0.0013888888947156122),
+          sconst(0.008333333333307118), sconst(0.04166666666651493), sconst(0.166666666666667),
+          sconst(0.5000000000000013)} {}
+};
+__device__ __forceinline__ double exp64(double y, const ExpConst &c) {
+  const double n = __builtin_rint(y * c.log2e);
+  double r = fma(n, c.ln2_hi, y);
+  r = fma(n, c.ln2_lo, r);
+  double q = c.q[0];
+#pragma unroll
+  for (int k = 1; k < 10; ++k) q = fma(q, r, c.q[k]);
+  q = fma(q, r, 1.0);
+  q = fma(q, r, 1.0);
+  return __builtin_amdgcn_ldexp(q, (int)n);
+}
+
 // Cosine and sine of x = w r in [0, pi] (up to 1e-4 beyond), as -sin and cos
 // of y = x - pi/2: odd and even polynomials in y (fit errors 2e-19, 6e-18).
 __device__ __forceinline__ double quarter_shift(double w, double r) {
@@ -1109,15 +1135,30 @@ __device__ __forceinline__ void ang_bwd_grid(const TripletList &tl, uint32_t q, 
     }
   } else {
     // from the LDS records: the lines' g contracted with the powers (sb) and
-    // with their cos-derivatives (sa), each sum started from its first term
+    // with their cos-derivatives (sa), each sum started from its first term.
+    // Long lists leave one wave per SIMD here (LDS), so what one wave waits for
+    // counts: a record is read whole before its use, two etas per trip, the
+    // exponential's constants once per triplet (FP64, eight etas, one wave per
+    // atom: 221 neighbours 2554 -> 2154 us, 449: 8377 -> 6690, 68: 204 -> 188).
+    typename std::conditional<sizeof(T) == 8, ExpConst, int>::type ec{};
+#pragma unroll 2
     for (int h = 0; h < sf.n_eta; ++h) {
       const T *rec = s_er + h * EtaRec<NZ>::RS;
-      const T E = exp_coef(rec[4 * NZ + 1], S2);
+      T gA[2 * NZ], gW[2 * NZ];
+#pragma unroll
+      for (int j = 0; j < 2 * NZ; ++j) {
+        gA[j] = rec[j];
+        gW[j] = rec[2 * NZ + j];
+      }
+      T E;
+      if constexpr (sizeof(T) == 8)
+        E = exp64(rec[4 * NZ + 1] * S2, ec);
+      else
+        E = exp_coef(rec[4 * NZ + 1], S2);
       T sa = 0, sb = 0;
 #pragma unroll
       for (int k = 0; k < NZ; ++k) {
-        const T gp = rec[k] + wab * rec[2 * NZ + k];
-        const T gm = rec[NZ + k] + wab * rec[3 * NZ + k];
+        const T gp = gA[k] + wab * gW[k], gm = gA[NZ + k] + wab * gW[NZ + k];
         sa = k == 0 ? gp * dPp[0] : fma(gp, dPp[k], sa);
         sb = k == 0 ? gp * Pp[0] : fma(gp, Pp[k], sb);
         sa = fma(gm, dPm[k], sa);
