@@ -101,8 +101,8 @@ def stage_kernel(stage, mixed, tune, z16, des_len, n_atoms, nsparse, c64=False, 
     n_atoms (grid-form tables with 4 zetas; z16: the zeta list is {1, 2, 4,
     16}; c64: the mixed run contracts in FP64; n_eta: etas of the table).  The
     backward's third argument is its form: 4 zetas, plus 10 where it holds five
-    to eight etas in registers (FP32) or 20 where it reads them from LDS (more
-    than eight, FP64 more than four).  The contraction is
+    to eight etas in registers (FP32) or 20 where it reads them from LDS (FP32
+    one, two and more than eight, FP64 more than four).  The contraction is
     instantiated for the descriptor length padded to 32; the mixed one as
     <bf16, D, row blocks per wave, waves>: four waves of one or two 16-row
     blocks up to 128 features, eight waves of one block above."""
@@ -113,7 +113,8 @@ def stage_kernel(stage, mixed, tune, z16, des_len, n_atoms, nsparse, c64=False, 
         return "k_desc_fwd_grid<%s, 4, %d, %s, false>" % (t, w, z), n_atoms * 64 * w
     if stage == "descriptors_bwd":
         w = tune["waves_bwd"]
-        form = 4 if n_eta <= 4 else 14 if mixed and n_eta <= 8 else 24
+        sets = 0 if mixed and n_eta <= 2 else 1 if n_eta <= 4 else 2 if mixed and n_eta <= 8 else 0
+        form = (24, 4, 14)[sets]
         return "k_desc_bwd<%s, %d, %d, %s, false>" % (t, w, form, z), n_atoms * 64 * w
     if stage == "gpr_contraction":
         dp = (des_len + 31) // 32 * 32

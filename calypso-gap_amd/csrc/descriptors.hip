@@ -1276,7 +1276,7 @@ __host__ __device__ constexpr int bwd_acc_doubles(const Lds &L) {
 
 // FORM: 0 the generic form; for grid tables of NZ zetas NZ, NZ + 10 or NZ + 20
 // with ES = 1, 2 or 0: at most 4 ES etas, whose g stays in registers
-// (ang_bwd_grid), or any number, read from LDS records.
+// (ang_bwd_grid), or any number, read from LDS records (bwd_sets).
 constexpr int bwd_form(int nz, int es) { return nz == 0 ? 0 : nz + (es == 1 ? 0 : es == 2 ? 10 : 20); }
 constexpr int form_sets(int form) { return form == 0 || form >= 20 ? 0 : form >= 10 ? 2 : 1; }
 //
@@ -1328,6 +1328,7 @@ __global__ __launch_bounds__(W > 4 ? 64 * W : 256, 2) void k_desc_bwd(int N, con
   // for its 2 NZ lines, so the radial and the angular regions together hold
   // at most 4 (n_rad + n_ang) <= 2 Dp values.
   constexpr int RS = EtaRec<GNZ>::RS;
+  static_assert(GNZ == 0 || RS == 4 * (GNZ + 1), "the record length in bwd_tables");
   static_assert(RS <= 8 * GNZ, "radial and eta records within 2 Dp values");
   T *s_er = s_gA;
 
@@ -1544,11 +1545,11 @@ size_t fwd_lds(const Lds &L) {
          (size_t)(6 * L.KP + (FG ? 0 : L.G * L.KP) + L.Dp + W * 2 * NCH) * sizeof(T);
 }
 
-// REGS: the register form of the grid backward, without angular g records.
+// tables: values of the backward's line tables (bwd_tables).
 template <typename T, int W, bool FG>
-size_t bwd_lds(const Lds &L, bool regs) {
+size_t bwd_lds(const Lds &L, int tables) {
   return (6 * W + (size_t)bwd_acc_doubles<T, W>(L)) * sizeof(double) +
-         (size_t)(6 * L.KP + (FG ? 0 : 2 * L.G * L.KP) + (regs ? 4 * L.n_rad : 2 * L.Dp)) * sizeof(T);
+         (size_t)(6 * L.KP + (FG ? 0 : 2 * L.G * L.KP) + tables) * sizeof(T);
 }
 
 // The layout that sets the longest accepted list: every other one is smaller.
@@ -1659,18 +1660,35 @@ bool zeta_1_2_4_16(const SFDev &sf) {
   return sf.nz == 4 && sf.zlog[0] == 0 && sf.zlog[1] == 1 && sf.zlog[2] == 2 && sf.zlog[3] == 4;
 }
 
-// Whether the backward keeps g in registers: a grid of at most four etas, or
-// in FP32 eight.
+// Sets of four etas whose g the backward of this table keeps in registers; 0:
+// from LDS records.  In FP32 three quarters or half of a set's matrix products
+// are zeros for one and two etas, and where long lists leave one wave per SIMD
+// nothing hides their time.  Registers and records there, us, one wave per atom:
+// one eta of four zetas 12,000 atoms of 63 neighbours 121 112, of 181 864 689;
+// of three 113 109, 778 696; of one 102 104, 626 620; two etas of four zetas 121
+// 121, 865 773 and 4096 atoms of 436 2396 2081; of five 130 133, 912 868 (but
+// 30,000 of 63 292 306), of three 114 117, 769 761, of two 111 114, 706 729, of
+// one 104 109, 632 659.
 template <typename T>
-bool bwd_regs(const SFDev &sf) {
-  return sf.grid && sf.n_eta <= (sizeof(T) == 4 ? 8 : 4);
+int bwd_sets(const SFDev &sf) {
+  if (!sf.grid) return 0;
+  if (sizeof(T) == 8) return sf.n_eta <= 4 ? 1 : 0;
+  if (sf.n_eta == 1 || (sf.n_eta == 2 && sf.nz == 4)) return 0;
+  return sf.n_eta <= 4 ? 1 : sf.n_eta <= 8 ? 2 : 0;
+}
+
+// Values of its line tables in LDS: radial records, then eta records or the
+// generic form's g (at most 2 Dp, see k_desc_bwd).
+template <typename T>
+int bwd_tables(const SFDev &sf) {
+  return 4 * sf.n_rad + (!sf.grid ? 2 * sf.n_ang : bwd_sets<T>(sf) > 0 ? 0 : sf.n_eta * 4 * (sf.nz + 1));
 }
 
 template <typename T, int W, int GNZ, bool Z16, bool FG, int ES>
 hipError_t bwd_launch_as(hipStream_t s, int N, const int *species, const double *wz, const NeighborBufs &nb,
                       const TripletBufs &tb, const SFDev &sf, Lds L, const GradSrc &gs, double *slot_f,
                       double *atom_vir) {
-  const size_t lds = bwd_lds<T, W, FG>(L, ES > 0);
+  const size_t lds = bwd_lds<T, W, FG>(L, bwd_tables<T>(sf));
   const hipError_t e = allow_lds((const void *)k_desc_bwd<T, W, bwd_form(GNZ, ES), Z16, FG>, lds);
   if (e != hipSuccess) return e;
   k_desc_bwd<T, W, bwd_form(GNZ, ES), Z16, FG><<<N, 64 * W, lds, s>>>(N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
@@ -1682,9 +1700,10 @@ hipError_t bwd_launch(hipStream_t s, int N, const int *species, const double *wz
                       const TripletBufs &tb, const SFDev &sf, Lds L, const GradSrc &gs, double *slot_f,
                       double *atom_vir) {
   if constexpr (GNZ > 0) {
-    if (sf.n_eta <= 4) return bwd_launch_as<T, W, GNZ, Z16, FG, 1>(s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
+    const int sets = bwd_sets<T>(sf);
+    if (sets == 1) return bwd_launch_as<T, W, GNZ, Z16, FG, 1>(s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
     if constexpr (sizeof(T) == 4)
-      if (sf.n_eta <= 8) return bwd_launch_as<T, W, GNZ, Z16, FG, 2>(s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
+      if (sets == 2) return bwd_launch_as<T, W, GNZ, Z16, FG, 2>(s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
   }
   return bwd_launch_as<T, W, GNZ, Z16, FG, 0>(s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);
 }
@@ -1760,7 +1779,7 @@ hipError_t fwd_grid(int waves, hipStream_t s, int N, const int *species, const d
 template <typename T>
 bool needs_global_tables(const SFDev &sf, const Lds &L) {
   const size_t lim = lds_limit();
-  if (bwd_lds<T, 1, false>(L, bwd_regs<T>(sf)) > lim) return true;
+  if (bwd_lds<T, 1, false>(L, bwd_tables<T>(sf)) > lim) return true;
   if (!sf.grid) return fwd_lds<T, 16, 1, false>(L) > lim;
   return fwd_grid_lds<T, 5, 1, false>(L) > lim;  // the widest grid layout
 }
@@ -1781,11 +1800,11 @@ hipError_t bwd_fit(int waves, hipStream_t s, int N, const int *species, const do
   int W;
   bool fg;
   auto bytes = [&](int w, bool g) {
-    const bool regs = bwd_regs<T>(sf);
-    if (w == 8) return bwd_lds<T, 8, false>(L, regs);
-    if (w == 4) return bwd_lds<T, 4, false>(L, regs);
-    if (w == 2) return bwd_lds<T, 2, false>(L, regs);
-    return g ? bwd_lds<T, 1, true>(L, regs) : bwd_lds<T, 1, false>(L, regs);
+    const int tables = bwd_tables<T>(sf);
+    if (w == 8) return bwd_lds<T, 8, false>(L, tables);
+    if (w == 4) return bwd_lds<T, 4, false>(L, tables);
+    if (w == 2) return bwd_lds<T, 2, false>(L, tables);
+    return g ? bwd_lds<T, 1, true>(L, tables) : bwd_lds<T, 1, false>(L, tables);
   };
   if (!pick_shape(waves, 8, bytes, W, fg) || (fg && !nb.fc_scratch)) return hipErrorInvalidValue;
   if (fg) return bwd_grid<T, 1, true>(s, N, species, wz, nb, tb, sf, L, gs, slot_f, atom_vir);

@@ -14,7 +14,8 @@ import bench  # noqa: E402
 from gapx import synth  # noqa: E402
 
 
-@pytest.mark.parametrize("n_eta,mixed,form", [(1, True, 4), (4, True, 4), (5, True, 14), (8, True, 14), (9, True, 24),
+@pytest.mark.parametrize("n_eta,mixed,form", [(1, True, 24), (2, True, 24), (3, True, 4), (4, True, 4),
+                                              (1, False, 4), (5, True, 14), (8, True, 14), (9, True, 24),
                                               (4, False, 4), (5, False, 24), (8, False, 24)])
 def test_backward_form_follows_the_etas(n_eta, mixed, form):
     t = {"waves_bwd": 2}
