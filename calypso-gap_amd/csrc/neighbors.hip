@@ -356,6 +356,12 @@ __device__ __forceinline__ float4 trip_record(double dx, double dy, double dz, d
 __host__ __device__ constexpr size_t trip_lds_records(int kcap) {
   return (size_t)std::max(kcap, std::min(kcap, 256) + std::min(kcap, 256) / 2);
 }
+// k_build's: behind the staged neighbours first the image search's records and
+// marks (kImageRecords), then, in the same place, the repeated half.
+constexpr int kImageRecords = 48;
+constexpr size_t build_lds_records(int kcap) {
+  return std::max(trip_lds_records(kcap), (size_t)kcap + kImageRecords);
+}
 
 // NARROW: 16-bit entries (lists of at most kNarrowSlots slots).  Half the bytes
 // of the list, which the wave's appends and the descriptor kernels' reads both
@@ -446,11 +452,14 @@ __device__ __forceinline__ void triplets_from_lds(int i, int K, float4 *s_p, dou
     };
     typedef std::integral_constant<int, 1> C1;
     typedef std::integral_constant<int, 2> C2;
+    typedef std::integral_constant<int, 3> C3;
     typedef std::integral_constant<int, 4> C4;
     if (K <= 64)
       runs(C1{}, C4{});
     else if (K <= 128)
       runs(C2{}, C2{});
+    else if (K <= 192)
+      runs(C3{}, C1{});
     else
       runs(C4{}, C1{});
   } else {
@@ -480,12 +489,15 @@ __device__ __forceinline__ void triplets_from_lds(int i, int K, float4 *s_p, dou
 }
 
 // A bin image that holds atoms: its first atom's slot less the candidates
-// before it, its lattice translation (three components of -64 .. 64 in bytes)
-// and that translation's vector.
+// before it, and its lattice translation (three components of -64 .. 64 in
+// bytes).  The translation's vector is formed again for each candidate: with it
+// in the record a long list's workgroup took 2.3 KB more LDS (4096 atoms of
+// 436 neighbours 758 -> 579 us; 12,000 of 181, three chunks of triplets instead
+// of four as well, 300 -> 262; ordinary lists the same).
 struct ImageRec {
   int first, t;
-  double sx, sy, sz;
 };
+static_assert(64 * (sizeof(ImageRec) + sizeof(int)) <= sizeof(float4) * kImageRecords, "the image search's place");
 
 // Order of LDS accesses within the one wave of a workgroup: the hardware keeps
 // it, the compiler has to be told.
@@ -512,9 +524,8 @@ __device__ __forceinline__ void wave_order() {
 template <bool TRIP>
 __device__ __forceinline__ int neighbour_list(int i, int lane, const int *__restrict__ atom_struct,
                                               const StructParams *__restrict__ sp, double rcut,
-                                              const NeighborBufs &nb, double rcA, float4 *s_p) {
-  __shared__ ImageRec s_rec[64];
-  __shared__ int s_flag[64];
+                                              const NeighborBufs &nb, double rcA, float4 *s_p, ImageRec *s_rec,
+                                              int *s_flag) {
   s_flag[lane] = 0;
   int mark = 0;
   const StructParams &P = sp[atom_struct[i]];
@@ -589,7 +600,7 @@ __device__ __forceinline__ int neighbour_list(int i, int lane, const int *__rest
     const int total = __builtin_amdgcn_readlane(incl, 63);
     const int excl = incl - n;
     // the group's bins that hold atoms, compacted in image order: candidate c of
-    // a bin sits at slot first + c, its atoms are shifted by the lattice vector
+    // a bin sits at slot first + c, its atoms are shifted by a lattice vector
     const unsigned long long held = __ballot(n > 0);
     const unsigned below =
         __builtin_amdgcn_mbcnt_hi((unsigned)(held >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)held, 0u));
@@ -597,9 +608,6 @@ __device__ __forceinline__ int neighbour_list(int i, int lane, const int *__rest
       ImageRec rec;
       rec.first = lo - excl;
       rec.t = (t0 + 64) | ((t1 + 64) << 8) | ((t2 + 64) << 16);
-      rec.sx = t0 * P.L[0] + t1 * P.L[3] + t2 * P.L[6];
-      rec.sy = t0 * P.L[1] + t1 * P.L[4] + t2 * P.L[7];
-      rec.sz = t0 * P.L[2] + t1 * P.L[5] + t2 * P.L[8];
       s_rec[below] = rec;
     }
     // candidate c0 + lane: its image's record and its atom's
@@ -641,9 +649,12 @@ __device__ __forceinline__ int neighbour_list(int i, int lane, const int *__rest
       double dx = 0, dy = 0, dz = 0, r = 0;
       if (c < total) {
         if (!(T0 == 0 && T1 == 0 && T2 == 0 && inf.x == i)) {
-          dx = pxy.x + rec.sx - xi;
-          dy = pxy.y + rec.sy - yi;
-          dz = pz + rec.sz - zi;
+          const double sx = T0 * P.L[0] + T1 * P.L[3] + T2 * P.L[6];
+          const double sy = T0 * P.L[1] + T1 * P.L[4] + T2 * P.L[7];
+          const double sz = T0 * P.L[2] + T1 * P.L[5] + T2 * P.L[8];
+          dx = pxy.x + sx - xi;
+          dy = pxy.y + sy - yi;
+          dz = pz + sz - zi;
           r = sqrt(dx * dx + dy * dy + dz * dz);
           ok = !(r > rcut);
         }
@@ -688,11 +699,13 @@ __global__ __launch_bounds__(64 * W) void k_build(int N, const int *__restrict__
                                                   const StructParams *__restrict__ sp, double rcut, NeighborBufs nb,
                                                   double rcA, TripletBufs tb) {
   extern __shared__ __align__(16) unsigned char smem[];
-  float4 *s_p = (float4 *)smem;  // [trip_lds_records(kcap)] with TRIP
+  float4 *s_p = (float4 *)smem;  // [build_lds_records(kcap)] with TRIP, else [kImageRecords]
+  ImageRec *s_rec = (ImageRec *)(s_p + (TRIP ? nb.kcap : 0));  // [64]
+  int *s_flag = (int *)(s_rec + 64);                           // [64]
   const int i = blockIdx.x, lane = threadIdx.x & 63;
   if (i >= N) return;
   if constexpr (W == 1) {
-    const int K = neighbour_list<TRIP>(i, lane, atom_struct, sp, rcut, nb, rcA, s_p);
+    const int K = neighbour_list<TRIP>(i, lane, atom_struct, sp, rcut, nb, rcA, s_p, s_rec, s_flag);
     if (TRIP) {
       __syncthreads();
       if (tb.narrow)
@@ -704,7 +717,7 @@ __global__ __launch_bounds__(64 * W) void k_build(int N, const int *__restrict__
     __shared__ int s_K;
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     if (wv == 0) {
-      const int K = neighbour_list<TRIP>(i, lane, atom_struct, sp, rcut, nb, rcA, s_p);
+      const int K = neighbour_list<TRIP>(i, lane, atom_struct, sp, rcut, nb, rcA, s_p, s_rec, s_flag);
       if (lane == 0) s_K = K;
     }
     __syncthreads();
@@ -1158,7 +1171,7 @@ static int build_waves(int N) { return N <= 768 ? 8 : N <= 1536 ? 4 : 1; }
 template <int W>
 static hipError_t launch_build(hipStream_t s, int N, const int *atom_struct, const StructParams *sp, double rcut,
                                const NeighborBufs &nb, double rcA, const TripletBufs &tb) {
-  const size_t lds = sizeof(float4) * trip_lds_records(nb.kcap);
+  const size_t lds = sizeof(float4) * build_lds_records(nb.kcap);
   k_build<true, W><<<N, 64 * W, lds, s>>>(N, atom_struct, sp, rcut, nb, rcA, tb);
   return hipGetLastError();
 }
@@ -1166,7 +1179,7 @@ static hipError_t launch_build(hipStream_t s, int N, const int *atom_struct, con
 hipError_t launch_build_neighbors(hipStream_t s, int N, const int *atom_struct, const StructParams *sp,
                                   double rcut, NeighborBufs nb, double rcA, const TripletBufs *tb) {
   if (!tb) {
-    k_build<false, 1><<<N, 64, 0, s>>>(N, atom_struct, sp, rcut, nb, 0.0, TripletBufs{});
+    k_build<false, 1><<<N, 64, sizeof(float4) * kImageRecords, s>>>(N, atom_struct, sp, rcut, nb, 0.0, TripletBufs{});
     return hipGetLastError();
   }
   switch (build_waves(N)) {
