@@ -694,7 +694,7 @@ static void default_tuning(Ctx &c) {
     // against 4926 but eager 5026 against 4938; 32,768 atoms with D = 256,
     // one workgroup a CU, 2186 against 2164, eager 2326 against 2150)
     t.halves = (!c64 && m.Dp <= 128) ? 1 : 0;
-    if (!c.waves_fwd_given) t.waves_fwd = default_waves_fwd(c.N, fp64);
+    if (!c.waves_fwd_given) t.waves_fwd = default_waves_fwd(fp64, m.sfd, m.Dp, c.kcap, c.N);
     if (!c.waves_bwd_given) t.waves_bwd = default_waves_bwd(c.N, fp64, grid);
     const int pts = gpr_points_per_chunk(m.Dp), chunks = m.Mp / pts;
     const double scale = m.Dp / 128.0 * pts / 64.0;
@@ -2010,7 +2010,7 @@ static int ctx_car2acsf(Ctx &c, int na, int max_nb, int nf, const double *pos, c
   o.Dp = Dp;
   // shapes by this table's size, as a load picks them by its batch's; those in
   // c.tune are the context's last evaluation's
-  const int waves_fwd = c.waves_fwd_given ? c.tune[0].waves_fwd : default_waves_fwd(N, true);
+  const int waves_fwd = c.waves_fwd_given ? c.tune[0].waves_fwd : default_waves_fwd(true, m.sfd, Dp, kcap, N);
   const int waves_bwd = c.waves_bwd_given ? c.tune[0].waves_bwd : default_waves_bwd(N, true, m.sfd.grid != 0);
   GAPX_HIP(launch_descriptors_fwd(c.stream, true, N, nullptr, m.d_wz, nb, tb, m.sfd, m.d_theta_inv, m.d_mu, 0, o,
                                   c.chunk > 0 ? c.chunk : 16, waves_fwd, kcap));

@@ -31,6 +31,7 @@
 // zeta), so exponentials, cutoff products and the powers (1 + lambda cos)^zeta
 // are updated incrementally along a chunk (zeta = 2, 4, 16 by squaring).
 #include <atomic>
+#include <cmath>
 #include <mutex>
 #include <set>
 #include <utility>
@@ -1827,6 +1828,25 @@ int max_neighbors_for_lds(bool fp64, const SFDev &sf, int Dp) {
     if (fp64 ? fits<double>(sf, L) : fits<float>(sf, L)) break;
   }
   return kp;
+}
+
+// A long list is worth several waves per atom whenever one each leaves a CU with
+// fewer waves than hide their latencies: about 8 in FP64, 16 in FP32.  How many
+// it has follows from the LDS (places) and from how N atoms fill the rounds.
+// One, two and four waves, us (places): FP64, 181 neighbours of seven cutoffs
+// (5) 4096 atoms 3860 2259 2311, 8000 7037 4460 4573; of one (10) 1500 463 456
+// 385, 3000 852 697 743, 4096 830 962 956, 8000 1681 1750 1868.  FP32, seven (11)
+// 4096 1433 1015 859; one (21) 1500 377 239 211, 3000 415 404 355, 4096 430 489
+// 440, 8000 820 829 833.  Lists of 95 stay with the waves their number asks for
+// (one cutoff, 3000 atoms: FP64 279 257 328, FP32 136 143 150).
+int default_waves_fwd(bool fp64, const SFDev &sf, int Dp, int KP, int N) {
+  const int waves = waves_within(N, fwd_wave_cap(fp64), 1);
+  if (sf.grid || KP < 192 || N <= 0) return waves;
+  const Lds L{KP, sf.n_groups > 0 ? sf.n_groups : 1, Dp, 0, sf.n_rad};
+  const size_t bytes = fp64 ? fwd_lds<double, 16, 1, false>(L) : fwd_lds<float, 16, 1, false>(L);
+  const double places = (double)std::max<size_t>(1, lds_limit() / bytes), atoms = N / 256.0;
+  const double in_flight = atoms / std::ceil(atoms / places);
+  return in_flight < (fp64 ? 7.5 : 15.0) ? std::max(waves, 4) : waves;
 }
 
 size_t desc_table_scratch_bytes(bool fp64, const SFDev &sf, int Dp, int KP, int N) {

@@ -330,7 +330,10 @@ constexpr int waves_within(int N, int cap, int least) {
     if ((long long)N * w <= cap) return w;
   return least;
 }
-constexpr int default_waves_fwd(int N, bool fp64) { return waves_within(N, fwd_wave_cap(fp64), 1); }
+// The generic forward takes four at longer lists too (KP slots per atom) where
+// the chip's rounds of one-wave workgroups would leave few waves on a CU, for LDS
+// or for want of atoms (default_waves_fwd in descriptors.hip).
+int default_waves_fwd(bool fp64, const SFDev &sf, int Dp, int KP, int N);
 constexpr int default_waves_bwd(int N, bool fp64, bool grid) {
   return waves_within(N, bwd_wave_cap(fp64, grid), grid ? 1 : 4);
 }
